@@ -318,6 +318,44 @@ def test_linear_f32_swiglu(pkg, oracle, cuda):
         np.testing.assert_allclose(y[r], ref, rtol=1e-4, atol=1e-4)
 
 
+# More than 8 rows run on fp32 MFMA: 64 x 64 tiles where there are at least 192 of them, else
+# 16 W rows x 16 / 32 / 64 rows of x per workgroup. Edges of both tiles and of the 32-k stages,
+# rows that start off 16-byte boundaries (k % 4), K parts of unequal and of no length.
+@pytest.mark.parametrize("m,n,k", [(9, 40, 4), (16, 16, 7), (17, 33, 95), (32, 100, 1000), (33, 64, 33),
+                                   (64, 50, 2052), (65, 48, 288), (200, 96, 31), (130, 8200, 66),
+                                   (64, 12289, 64), (769, 1040, 36), (1000, 1000, 4097)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_linear_f32_many_rows(pkg, cuda, m, n, k, swiglu):
+    import torch
+    n = n // 16 * 16 if swiglu else n
+    g = torch.Generator(device=cuda).manual_seed(m + n + k)
+    w = torch.randn((n, k), generator=g, device=cuda)
+    x = torch.randn((m, k), generator=g, device=cuda)
+    x[m // 2] *= 1e30  # a row's scale does not touch its neighbours
+    bias = torch.randn(n, generator=g, device=cuda)
+    tw = pkg.TiledWeight("f32", n, k, w.view(-1).view(torch.uint8), pkg.weight_layout("f32", n, k))
+    # a chain of additions loses at most 2^-24 of the sum of magnitudes per addition: 32 in a
+    # stage, 8 stages, then one per 256 k, the K parts and the bias
+    grow = (32 + 8 + k / 256 + 8 + 2) * 2.0 ** -24
+    w64, x64 = w.double(), x.double()
+    ref = x64 @ w64.t().contiguous() + bias.double()
+    bound = grow * (x64.abs() @ w64.abs().t().contiguous() + bias.abs().double())
+    y = pkg.linear(tw, x, bias=bias, act=pkg.EPI_SWIGLU if swiglu else pkg.EPI_NONE).double()
+    if not swiglu:
+        assert bool(((y - ref).abs() <= bound).all())
+        return
+    t = ref.view(m, n // 16, 2, 8)
+    e = bound.view(m, n // 16, 2, 8)
+    gate, up = t[:, :, 0], t[:, :, 1]
+    want = torch.nn.functional.silu(gate) * up
+    # |silu'| <= 1.1, |silu(g)| <= |g|; fp32 exp, divide and products: 16 ulp
+    slack = 1.1 * e[:, :, 0] * up.abs() + gate.abs() * e[:, :, 1] + e[:, :, 0] * e[:, :, 1] * 1.1
+    slack = slack + 16 * 2.0 ** -23 * (gate * up).abs() + 1e-30
+    finite = (gate * up).abs() < 1e38  # the scaled row's products leave fp32
+    got = y.view(m, n // 16, 8)
+    assert bool(((got - want).abs() <= slack)[finite].all())
+
+
 # ---- argmax ------------------------------------------------------------------------------
 def test_argmax(pkg, oracle, cuda):
     import torch
