@@ -143,8 +143,10 @@ __device__ __forceinline__ f4_t load_row4(rsrc_t r, uint32_t row_off, int col, i
 // ---- 64 x 64 output tiles ---------------------------------------------------
 // KS groups of four waves; group ks takes the ks-th part of K, its waves the
 // tile's four 32 x 32 quarters (v_mfma_f32_32x32x2_f32). A stage is 32 k of 64
-// x rows and 64 W rows, 16-byte loads of 128 contiguous bytes per row, one
-// stage ahead in registers, two LDS slabs, one barrier per stage. Lane half h
+// x rows and 64 W rows, 16-byte loads of 128 contiguous bytes per row, two
+// stages ahead in registers (one stage's MFMAs, ~0.5 us, are shorter than a
+// trip to HBM: 95 us with one at 200 x 4096 x 4096, 77 with two), two LDS
+// slabs, one barrier per stage. Lane half h
 // of a fragment reads k = 8j + 4h .. +3 as one 16-byte LDS read and feeds
 // four MFMAs, whose k pair is (8j + i, 8j + 4 + i): any pairing covers the
 // sum. Rows are padded to 36 floats, which spreads those reads over the banks.
@@ -179,15 +181,15 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_kernel(F32Args a) {
   const int t = tid & 255;
   const int lrow = t >> 3, lcol = 4 * (t & 7);
   float* slab = smem + ks * 2 * 2 * kTile * kLdsRow;
-  f4_t pre[4];
-  auto load = [&](int s) __attribute__((always_inline)) {
+  f4_t even[4], odd[4];
+  auto load = [&](f4_t (&pre)[4], int s) __attribute__((always_inline)) {
     const int col = k0 + s * kStageK + lcol;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       pre[i] = load_row4<VEC>(i < 2 ? rx : rw,
                               (uint32_t)(((i & 1) * 32 + lrow) * a.k) * 4, col, kend);
   };
-  auto store = [&](int buf) __attribute__((always_inline)) {
+  auto store = [&](const f4_t (&pre)[4], int buf) __attribute__((always_inline)) {
     float* p = slab + buf * 2 * kTile * kLdsRow;
 #pragma unroll
     for (int i = 0; i < 4; ++i) *(f4_t*)(p + (i * 32 + lrow) * kLdsRow + lcol) = pre[i];
@@ -195,12 +197,8 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_kernel(F32Args a) {
   f16v_t sum = {}, mid = {};
   const int frag = (lane & 31) * kLdsRow + 4 * (lane >> 5);
   const int arow = 32 * wm * kLdsRow + frag, brow = (kTile + 32 * wn) * kLdsRow + frag;
-  load(0);
-  store(0);
-  for (int s = 0; s < per_ks; ++s) {
-    if (s + 1 < per_ks) load(s + 1);
-    __syncthreads();
-    const float* p = slab + (s & 1) * 2 * kTile * kLdsRow;
+  auto run = [&](int buf) __attribute__((always_inline)) {
+    const float* p = slab + buf * 2 * kTile * kLdsRow;
     f16v_t in = {};
 #pragma unroll
     for (int j = 0; j < kStageK / 8; ++j) {
@@ -209,9 +207,23 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_kernel(F32Args a) {
       for (int i = 0; i < 4; ++i)
         in = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], in, 0, 0, 0);
     }
-    if (s + 1 < per_ks) store((s + 1) & 1);
     mid += in;
-    if ((s & 7) == 7) {
+  };
+  // stages past the part's end (an odd count, or the last prefetches) load
+  // zeros and add nothing
+  load(even, 0);
+  load(odd, 1);
+  store(even, 0);
+  for (int s = 0; s < per_ks; s += 2) {
+    load(even, s + 2);
+    __syncthreads();
+    run(0);
+    store(odd, 1);
+    load(odd, s + 3);
+    __syncthreads();
+    run(1);
+    store(even, 0);
+    if ((s & 6) == 6) {
       sum += mid;
       mid = (f16v_t){};
     }
