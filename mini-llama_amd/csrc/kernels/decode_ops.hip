@@ -1014,23 +1014,280 @@ __global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(At
   }
 }
 
-// Pass 2, per (query head, query row): four waves each take 16 chunks of a
-// 64-chunk pass. The partials' addresses do not depend on the position, so
-// the first pass requests every maximum, sum and accumulator (in bounds:
+// e^(s - m) for s <= m as 2^h (1 + f ln 2), h + f = (s - m) log2 e with h the
+// rounded product and f what it lost (log2 e in two parts): the hardware
+// exp2's own error and no more.
+__device__ __forceinline__ float exp_diff(float s, float m) {
+  constexpr float kLog2e = 1.44269504088896341f, kLn2 = 0.693147180559945309f;
+  constexpr float kLog2eLow = (float)(1.44269504088896340735992 - (double)kLog2e);
+  const float t = s - m, h = t * kLog2e;
+  const float f = __builtin_fmaf(t, kLog2eLow, __builtin_fmaf(t, kLog2e, -h));
+  const float e = __builtin_amdgcn_exp2f(h);
+  return h > -200.0f ? __builtin_fmaf(e * kLn2, f, e) : 0.0f;  // (-inf: f is NaN)
+}
+
+// ---- long caches: keys streamed through fp32 MFMA ----------------------------------
+// attn_reg_kernel gives every 32 positions a workgroup and a partial. At long
+// contexts that grid is many times the chip and its combine reads one partial
+// per 32 positions and head; its scores and P.V also take ~600 VALU per 8
+// positions and wave. Here a workgroup runs over every chunks-th span of
+// 16 W positions, a wave over 16 keys at a time with the next 16 keys' rows
+// in flight, and both products run on v_mfma_f32_16x16x4_f32 (exact fp32
+// products) with the group's query heads as the 16 rows (padding heads are
+// zero and never stored). K and V go straight from the cache to the B operand:
+//  - K: lane (key lane % 16, quarter ak = lane / 16) holds dims 16 s + 4 ak
+//    .. + 3, one 16-byte load per s (16 keys x 64 contiguous bytes); q is read
+//    in the same order, so the sum covers every dim once.
+//  - V: for keys 4 st + ak, dims 64 u + 4 (lane % 16) .. + 3 in one 16-byte
+//    load; component i feeds output tile (u, i), whose column j is dim
+//    64 u + 4 j + i.
+// Strided spans keep a short sequence in a long cache on many workgroups.
+// Bound by the reads of K and V.
+template <int HD, bool FUSED>
+__global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_stream_kernel(AttnArgs a) {
+  constexpr int W = prefill_waves(HD);
+  constexpr int KS = HD / 16;   // 16-byte pieces of K per lane
+  constexpr int VU = HD / 64;   // 16-byte pieces of V per lane and key
+  constexpr int QS = HD + 4;    // padded LDS row
+  constexpr int PS = 20;
+  constexpr bool AHEAD = HD <= 128;  // the next keys' rows fit the registers
+  // merge area: per wave 16 rows of acc; q and P live there before
+  __shared__ __align__(16) float lds[W * 16 * QS];
+  __shared__ float wm[W][16], wl[W][16];
+  __shared__ __align__(16) float kcur[FUSED ? HD : 4], vcur[FUSED ? HD : 4];
+  static_assert(16 * QS + W * 16 * PS <= W * 16 * QS, "q and P fit the merge area");
+
+  const int pos = read_scalar(a.pos_dev, a.pos);
+  const int len = pos + 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int chunk = blockIdx.x;
+  if (pos < 0 || pos >= a.pos_limit || chunk * (16 * W) >= len) return;
+  const int kvh = blockIdx.y;
+  const int G = a.group;
+  const int ai = lane & 15, ak = lane >> 4;
+  const size_t row_stride = (size_t)a.n_kv * HD;
+  const size_t cbase = (size_t)a.layer * a.max_seq * row_stride + (size_t)kvh * HD;
+  // rows past the range read as zeros; with a fused cache write the current
+  // row is not there yet and comes from k_new / v_new
+  const uint32_t rs4 = (uint32_t)row_stride * 4u;
+  const int rows = FUSED ? pos : len;
+  const uint32_t kvbytes = rows > 0 ? (uint32_t)(rows - 1) * rs4 + HD * 4u : 0u;
+  const rsrc_t rk = make_rsrc(a.keys + cbase, kvbytes);
+  const rsrc_t rv = make_rsrc(a.values + cbase, kvbytes);
+
+  struct Keys {
+    f4_t k[KS], v[4][VU];
+  };
+  auto load = [&](Keys& r, int k0) __attribute__((always_inline)) {
+    const uint32_t ko = (uint32_t)(k0 + ai) * rs4 + (uint32_t)ak * 16u;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) r.k[s] = __builtin_bit_cast(f4_t, buf_load16(rk, ko + 64u * s, 0));
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      const uint32_t vo = (uint32_t)(k0 + 4 * st + ak) * rs4 + (uint32_t)ai * 16u;
+#pragma unroll
+      for (int u = 0; u < VU; ++u)
+        r.v[st][u] = __builtin_bit_cast(f4_t, buf_load16(rv, vo + 256u * u, 0));
+    }
+  };
+  const int step = a.chunks * (16 * W);
+  int k0 = chunk * (16 * W) + wave * 16;
+  // the group's q rows, zero past G: their inputs are requested ahead of the
+  // K / V rows (loads return in order)
+  constexpr int QN = 16 * HD / (W * 64), QA = AHEAD ? QN : 0;
+  float qx[QA + 1], qy[QA + 1], qc[QA + 1], qsn[QA + 1];
+  auto q_inputs = [&](int e, float& x0, float& x1, float& c, float& sn) __attribute__((always_inline)) {
+    const int g = e / HD, d = e % HD;
+    const float* x = a.q + (size_t)(kvh * G + min(g, G - 1)) * HD;
+    x0 = x[d];
+    if constexpr (FUSED) {  // x * c + partner * sn
+      constexpr int H = HD / 2;
+      const bool first = a.neox ? d < H : (d & 1) == 0;
+      const int ii = a.neox ? (d < H ? d : d - H) : (d >> 1);
+      x1 = x[a.neox ? (first ? d + H : d - H) : d ^ 1];
+      c = a.rope_cs[ii];
+      sn = first ? -a.rope_cs[H + ii] : a.rope_cs[H + ii];
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < QA; ++i) q_inputs(threadIdx.x + i * W * 64, qx[i], qy[i], qc[i], qsn[i]);
+  Keys cur;
+  load(cur, k0);
+
+  float* qs = lds;
+#pragma unroll
+  for (int i = 0; i < QN; ++i) {
+    const int e = threadIdx.x + i * W * 64, j = AHEAD ? i : 0;
+    if constexpr (!AHEAD) q_inputs(e, qx[0], qy[0], qc[0], qsn[0]);
+    float v = qx[j];
+    if constexpr (FUSED) v = v * qc[j] + qy[j] * qsn[j];
+    qs[e / HD * QS + e % HD] = e / HD < G ? v : 0.0f;
+  }
+  if constexpr (FUSED) {
+    // the workgroup whose spans hold pos keeps its rotated k and its v, and
+    // writes the cache row
+    if (pos / (16 * W) % a.chunks == chunk) {
+      const size_t row = (((size_t)a.layer * a.max_seq + pos) * a.n_kv + kvh) * HD;
+      for (int d = threadIdx.x; d < HD; d += W * 64) {
+        const float kd = rope_elem<HD>(a.k_new + (size_t)kvh * HD, d, a.neox, a.rope_cs);
+        const float vd = a.v_new[(size_t)kvh * HD + d];
+        a.kc[row + d] = kcur[d] = kd;
+        a.vc[row + d] = vcur[d] = vd;
+      }
+    }
+  }
+  __syncthreads();
+  f4_t qa[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) qa[s] = *(const f4_t*)(qs + ai * QS + 16 * s + 4 * ak);
+  float* pw = lds + 16 * QS + wave * 16 * PS;
+
+  float m[4], l[4];  // rows 4 ak + i; l holds this lane's key column only
+  f4_t acc[4 * VU];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m[i] = -INFINITY;
+    l[i] = 0.0f;
+  }
+#pragma unroll
+  for (int t = 0; t < 4 * VU; ++t) acc[t] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+  auto run = [&](Keys& cur, int k0) __attribute__((always_inline)) {
+    if constexpr (FUSED) {
+      if (k0 + 16 > pos) {  // the span holding the current position
+        if (k0 + ai == pos) {
+#pragma unroll
+          for (int s = 0; s < KS; ++s) cur.k[s] = *(const f4_t*)(kcur + 16 * s + 4 * ak);
+        }
+#pragma unroll
+        for (int st = 0; st < 4; ++st)
+          if (k0 + 4 * st + ak == pos) {
+#pragma unroll
+            for (int u = 0; u < VU; ++u) cur.v[st][u] = *(const f4_t*)(vcur + 64 * u + 4 * ai);
+          }
+      }
+    }
+    // eight chains of HD / 32 MFMAs each, added as a tree: no more roundings
+    // on the way to a score than the register kernel's lane sums
+    f4_t sc8[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sc8[i] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f4_t& c = sc8[4 * (s & 1) + i];
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[s][i], cur.k[s][i], c, 0, 0, 0);
+      }
+    const f4_t sacc = ((sc8[0] + sc8[1]) + (sc8[2] + sc8[3])) + ((sc8[4] + sc8[5]) + (sc8[6] + sc8[7]));
+    const bool seen = k0 + ai < len;
+    float al[4];
+    bool rescale = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float sc = seen ? sacc[i] * a.scale : -INFINITY;
+      const float mx = fmaxf(m[i], row_max<16>(sc));
+      // (mx stays -inf only on rows whose scores are all -inf or NaN)
+      al[i] = mx == -INFINITY ? 1.0f : exp_diff(m[i], mx);
+      const float p = seen ? exp_diff(sc, mx) : 0.0f;
+      l[i] = l[i] * al[i] + p;
+      m[i] = mx;
+      rescale |= al[i] != 1.0f;
+      pw[(4 * ak + i) * PS + ai] = p;
+    }
+    if (__any(rescale)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < 4 * VU; ++t) acc[t][i] *= al[i];
+    }
+    // P from the D layout to the A layout through the wave's own LDS
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float pa[4];
+#pragma unroll
+    for (int st = 0; st < 4; ++st) pa[st] = pw[ai * PS + 4 * st + ak];
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+      for (int u = 0; u < VU; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[4 * u + i] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(pa[st], cur.v[st][u][i], acc[4 * u + i], 0, 0, 0);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // P is read before the next keys' weights
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  for (; k0 < len; k0 += step) {
+    if constexpr (AHEAD) {
+      Keys next;
+      load(next, k0 + step);  // (past the range: zeros, no traffic)
+      run(cur, k0);
+      cur = next;
+    } else {
+      run(cur, k0);
+      load(cur, k0 + step);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) l[i] = row_sum<16>(l[i]);
+
+  // the waves' partials merged in wave order
+  __syncthreads();  // q and P are done with: the merge area reuses them
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int u = 0; u < VU; ++u)
+      *(f4_t*)(lds + (wave * 16 + 4 * ak + i) * QS + 64 * u + 4 * ai) =
+          f4_t{acc[4 * u][i], acc[4 * u + 1][i], acc[4 * u + 2][i], acc[4 * u + 3][i]};
+    if (ai == 0) {
+      wm[wave][4 * ak + i] = m[i];
+      wl[wave][4 * ak + i] = l[i];
+    }
+  }
+  __syncthreads();
+  const Partials pp = partials_of(a, 0);
+  for (int e = threadIdx.x; e < G * HD; e += W * 64) {
+    const int g = e / HD, d = e - g * HD;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < W; ++w) mx = fmaxf(mx, wm[w][g]);
+    float sum = 0.0f, o = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float f = wm[w][g] == -INFINITY ? 0.0f : exp_diff(wm[w][g], mx);
+      // (a wave without keys holds zeros)
+      sum += wl[w][g] * f;
+      o += lds[(w * 16 + g) * QS + d] * f;
+    }
+    const size_t slot = (size_t)(kvh * G + g) * a.chunks + chunk;
+    if (d == 0) {
+      pp.m[slot] = mx;
+      pp.l[slot] = sum;
+    }
+    pp.acc[slot * HD + d] = o;
+  }
+}
+
+// Pass 2, per (query head, query row): each wave takes 16 chunks of a pass of
+// 64 (four waves) or 128 (eight: a 7B layer at position 8000 of 8192, 256
+// partials, 70.0 -> 66.5 us). The partials' addresses do not depend on the
+// position, so the first pass requests every maximum, sum and accumulator (in bounds:
 // chunks < a.chunks) together with the device position: one memory round
 // trip instead of four dependent ones. Chunks past the live range are
 // masked by selects after the loads (stale partials never enter a product).
-// Each wave rescales its chunks to its own maximum in chunk order; the four
+// Each wave rescales its chunks to its own maximum in chunk order; the
 // waves then merge through LDS in wave order, and passes in pass order
 // (deterministic).
-constexpr int kCombineWaves = 4;
 constexpr int kCombineCpw = 16;  // chunks per wave and pass
-constexpr int kCombinePass = kCombineWaves * kCombineCpw;
 
-// KD: head dims per lane (head_dim <= 64 KD)
-template <int KD>
-__global__ __launch_bounds__(kCombineWaves * 64) void attn_combine_kernel(AttnArgs a) {
-  constexpr int kD = KD;
+// KD: head dims per lane (head_dim <= 64 KD); W waves
+template <int KD, int W>
+__global__ __launch_bounds__(W * 64) void attn_combine_kernel(AttnArgs a) {
+  constexpr int kD = KD, kCombineWaves = W, kCombinePass = W * kCombineCpw;
   __shared__ float sm[kCombineWaves], sl[kCombineWaves];
   __shared__ float sacc[kCombineWaves][kAttnMaxHd];
   const int qrow = blockIdx.y;
@@ -1067,7 +1324,7 @@ __global__ __launch_bounds__(kCombineWaves * 64) void attn_combine_kernel(AttnAr
     }
     if constexpr (FIRST) {
       const int pos = read_scalar(a.pos_dev, a.pos) + qrow;
-      live = pos < 0 || pos >= a.pos_limit ? -1 : (pos + a.chunk_len) / a.chunk_len;
+      live = pos < 0 || pos >= a.pos_limit ? -1 : min((pos + a.chunk_len) / a.chunk_len, a.chunks);
     }
     if (live < 0) return;
     float wmx = -INFINITY;
@@ -1088,7 +1345,7 @@ __global__ __launch_bounds__(kCombineWaves * 64) void attn_combine_kernel(AttnAr
         for (int j = 0; j < kD; ++j) wacc[j] += (cw + i < live ? v[i][j] : 0.0f) * f;
       }
     }
-    // the four waves merged in wave order, then into the running result
+    // the waves merged in wave order, then into the running result
     __syncthreads();  // (a previous pass's readers are done with the LDS)
     if (lane == 0) {
       sm[wave] = wmx;
@@ -1526,6 +1783,24 @@ static void attn_launch_g(const AttnArgs& a, hipStream_t stream) {
   else if constexpr (HD != 64) attn_launch<HD, 16>(a, stream);
 }
 
+template <int HD>
+static void stream_launch(const AttnArgs& a, hipStream_t stream) {
+  const dim3 grid(a.chunks, a.n_kv), block(prefill_waves(HD) * 64);
+  if (a.rope_cs != nullptr)
+    hipLaunchKernelGGL((attn_stream_kernel<HD, true>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((attn_stream_kernel<HD, false>), grid, block, 0, stream, a);
+}
+
+template <int KD>
+static void combine_launch(const AttnArgs& a, int n_heads, hipStream_t stream) {
+  const dim3 grid(n_heads, a.rows);
+  if (a.chunks <= 4 * kCombineCpw)
+    hipLaunchKernelGGL((attn_combine_kernel<KD, 4>), grid, dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL((attn_combine_kernel<KD, 8>), grid, dim3(512), 0, stream, a);
+}
+
 // Query-head split of the register kernel: MLQ_ATTN_HSPLIT (read once)
 // overrides the rule in launch_attention.
 int attn_hsplit_override() {
@@ -1589,20 +1864,47 @@ hipError_t launch_attention(const AttnLaunch& r, hipStream_t stream) {
       a.hsplit = (a.group + a.hper - 1) / a.hper;  // no empty split
     }
   }
-  switch (reg ? r.hd : 0) {
-    case 64: attn_launch_g<64>(a, stream); break;
-    case 128: attn_launch_g<128>(a, stream); break;
-    case 256: attn_launch_g<256>(a, stream); break;
-    default: attn_launch_g<0>(a, stream); break;
+  // Long: the keys stream through attn_stream_kernel, two workgroups per CU.
+  // Position 30000 of a 32768 cache, 28 heads on 4 kv heads of 128 (123 MB):
+  // 65.9 -> 32.3 us with its combine (a chunk per workgroup left 938
+  // partials per head, and their combine took longer than the chunks); one
+  // workgroup per CU is the same, three 39.9. The line is 192 positions x kv
+  // heads per CU: below it the register kernel's finer chunks win (32 heads
+  // on 8 kv heads of 128, position 4200: 17.9 us against 18.6; 8000: 25.1
+  // against 20.6). A device position says only the capacity, so there
+  // more than 256: a 7B layer in a 32768 cache takes 0.15 us more at position
+  // 1100 and 33 us less at 30000.
+  const bool stream_keys = reg && a.rows == 1 && a.hsplit == 1 &&
+                           (int64_t)r.max_len * a.n_kv >
+                               (r.pos_dev != nullptr ? 256 : 192) * (int64_t)device_cus() &&
+                           (uint64_t)r.max_seq * r.n_kv * r.hd * 4 < (1ull << 31);
+  if (stream_keys) {
+    a.chunk_len = 16 * prefill_waves(r.hd);
+    // the same number of spans for every workgroup
+    const int spans = (r.max_len + a.chunk_len - 1) / a.chunk_len;
+    const int each = (spans + std::max(2 * device_cus() / a.n_kv, 16) - 1) /
+                     std::max(2 * device_cus() / a.n_kv, 16);
+    a.chunks = (spans + each - 1) / each;
+    switch (r.hd) {
+      case 64: stream_launch<64>(a, stream); break;
+      case 128: stream_launch<128>(a, stream); break;
+      default: stream_launch<256>(a, stream); break;
+    }
+  } else {
+    switch (reg ? r.hd : 0) {
+      case 64: attn_launch_g<64>(a, stream); break;
+      case 128: attn_launch_g<128>(a, stream); break;
+      case 256: attn_launch_g<256>(a, stream); break;
+      default: attn_launch_g<0>(a, stream); break;
+    }
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const dim3 cgrid(r.n_heads, a.rows), cblock(kCombineWaves * 64);
   switch ((r.hd + 63) / 64) {
-    case 1: hipLaunchKernelGGL(attn_combine_kernel<1>, cgrid, cblock, 0, stream, a); break;
-    case 2: hipLaunchKernelGGL(attn_combine_kernel<2>, cgrid, cblock, 0, stream, a); break;
-    case 3: hipLaunchKernelGGL(attn_combine_kernel<3>, cgrid, cblock, 0, stream, a); break;
-    default: hipLaunchKernelGGL(attn_combine_kernel<4>, cgrid, cblock, 0, stream, a); break;
+    case 1: combine_launch<1>(a, r.n_heads, stream); break;
+    case 2: combine_launch<2>(a, r.n_heads, stream); break;
+    case 3: combine_launch<3>(a, r.n_heads, stream); break;
+    default: combine_launch<4>(a, r.n_heads, stream); break;
   }
   return hipGetLastError();
 }

@@ -237,6 +237,64 @@ def test_attention_matches_oracle(pkg, oracle, cuda, n_heads, n_kv, hd, max_seq,
                                atol=1e-5)
 
 
+# Long caches stream their keys (more than 192 positions x kv heads per CU, 256 where the
+# position is on the device): spans of 64 positions (32 at head_dim 256) shared out over the workgroups, so positions
+# at the edges of 16-key steps, of spans and of a workgroup's second span; groups of 1 to 16 heads.
+@pytest.mark.parametrize("n_heads,n_kv,hd,max_seq,pos", [
+    (28, 4, 128, 13000, 12287), (28, 4, 128, 13000, 12288), (8, 8, 64, 7000, 6207), (32, 8, 64, 9000, 8207),
+    (64, 4, 128, 13000, 12415), (16, 1, 256, 50000, 49200), (40, 8, 256, 6300, 6159), (12, 2, 128, 25000, 24591)])
+def test_attention_long_cache(pkg, cuda, n_heads, n_kv, hd, max_seq, pos):
+    import torch
+    g = torch.Generator(device=cuda).manual_seed(pos)
+    keys = torch.randn((2, max_seq, n_kv, hd), generator=g, device=cuda)
+    values = torch.randn((2, max_seq, n_kv, hd), generator=g, device=cuda)
+    keys[:, pos + 1:] = float("nan")  # nothing past the position is used
+    values[:, pos + 1:] = float("nan")
+    q = torch.randn((n_heads, hd), generator=g, device=cuda)
+    c = pkg.MlqKvCache(keys.data_ptr(), values.data_ptr(), 2, max_seq, n_kv, hd)
+    lib = pkg.lib()
+    nbytes = ctypes.c_size_t()
+    _ok(pkg, lib.mlq_attention_workspace(ctypes.byref(c), n_heads, ctypes.byref(nbytes)), "ws")
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device=cuda)
+    out = torch.empty((n_heads, hd), device=cuda)
+    _ok(pkg, lib.mlq_attention_decode(ctypes.byref(c), 1, pos, q.data_ptr(), n_heads, out.data_ptr(),
+                                      ws.data_ptr(), ws.numel(), _s(pkg)), "attention")
+    k64 = keys[1, :pos + 1].double().repeat_interleave(n_heads // n_kv, dim=1)
+    v64 = values[1, :pos + 1].double().repeat_interleave(n_heads // n_kv, dim=1)
+    p = torch.softmax((k64 * q.double()).sum(dim=2) / hd ** 0.5, dim=0)
+    ref = (p[:, :, None] * v64).sum(dim=0)
+    # scores of about 1 to 2^-22 each way, weights and their sums in fp32
+    bound = 2e-6 * (p[:, :, None] * v64.abs()).sum(dim=0)
+    assert bool(((out.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("hd,n_heads,n_kv", [(64, 16, 16), (128, 56, 8), (256, 8, 8)])
+def test_decode_step_in_a_long_cache(pkg, cuda, hd, n_heads, n_kv):
+    """The device-position step (its grid covers the whole cache, so keys stream and the current row
+    is rotated and written by the streaming kernel) against the host-position step."""
+    import mini_llama_amd.decode as dec
+    from synthetic import synth
+    import torch
+    cfg = dict(vocab_size=200, dim=256, hidden_dim=256, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv,
+               head_dim=hd, max_seq_len=9000, rope_type=1)
+    model = synth.synthetic_model(cfg, "q8_0", seed=4)
+    host, device = dec.DecodeModel(model), dec.DecodeModel(model)
+    g = torch.Generator(device=cuda).manual_seed(hd)
+    host.keys.normal_(generator=g)
+    host.values.normal_(generator=g)
+    for pos in (0, 1, 15, 16, 63, 64, 8191, 8192, 8999):
+        device.keys.copy_(host.keys)
+        device.values.copy_(host.values)
+        want = host.forward_token(17, pos).clone()
+        device.token_dev.fill_(17)
+        device.pos_dev.fill_(pos)
+        device.step_device()
+        # the two orders of fp32 sums differ by ulps; nothing else does
+        assert float((device.logits - want).abs().max()) <= 2e-5 * float(want.abs().max()), pos
+        assert float((device.keys - host.keys).abs().max()) <= 2e-5, pos
+        assert float((device.values - host.values).abs().max()) <= 2e-5, pos
+
+
 @pytest.mark.parametrize("hd", [64, 128, 256])
 def test_attention_unaligned_buffers(pkg, oracle, cuda, hd):
     """Caches and q that are not 16-byte aligned take the LDS-staged kernel
