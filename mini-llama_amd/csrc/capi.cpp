@@ -67,6 +67,15 @@ bool uses_gemv(const mlq_weight* w, int m) {
   return m <= kGemvMaxRows && w->k <= gemv_max_k(w->type, m);
 }
 
+// 2..16 rows with x resident in LDS: shapes where that is the faster kernel,
+// and up to 8 rows too long for the GEMV's staging (the tuning overrides
+// name the other kernels' plans, so they keep those kernels).
+bool uses_rows(const mlq_weight* w, int m) {
+  if (m < 2 || m > 16 || (m <= kGemvMaxRows ? gemv_split_set() : skinny_plan_set())) return false;
+  if (!rows_supported(w->type, m, w->n, w->k)) return false;
+  return rows_faster(m, w->n, w->k) || (m <= kGemvMaxRows && !uses_gemv(w, m));
+}
+
 }  // namespace
 
 namespace mlq {
@@ -224,6 +233,8 @@ int mlq_linear_path(const mlq_weight* w, const float* x, float* y, int m,
     return hip_status(
         launch_linear_f32((const float*)w->base, w->n, w->k, x, y, m, (hipStream_t)stream));
   }
+  if (path == MLQ_PATH_AUTO && uses_rows(w, m))
+    return hip_status(launch_rows(*w, x, y, m, (hipStream_t)stream));
   const bool gemv_fits = uses_gemv(w, m);
   bool use_gemv;
   switch (path) {
@@ -250,7 +261,7 @@ int mlq_linear_workspace(const mlq_weight* w, int m, size_t* bytes) {
   if (rc != MLQ_OK) return rc;
   if (bytes == nullptr) return MLQ_ERR_INVALID_ARG;
   if (m <= 0) return MLQ_ERR_SHAPE;
-  *bytes = w->type == MLQ_F32 || uses_gemv(w, m) ? 0
+  *bytes = w->type == MLQ_F32 || uses_gemv(w, m) || uses_rows(w, m) ? 0
            : m <= kSkinnyMaxRows ? skinny_workspace_bytes(w->type, m, w->n, w->k)
                                  : gemm_workspace_bytes(m, w->n, w->k);
   return MLQ_OK;
@@ -271,6 +282,7 @@ int mlq_linear_epi(const mlq_weight* w, const float* x, float* y, int m,
   const hipStream_t s = (hipStream_t)stream;
   if (w->type == MLQ_F32)
     return hip_status(launch_linear_f32((const float*)w->base, w->n, w->k, x, y, m, s, epi));
+  if (uses_rows(w, m)) return hip_status(launch_rows(*w, x, y, m, s, epi));
   if (uses_gemv(w, m)) return hip_status(launch_gemv(*w, x, y, m, s, epi));
   const size_t need = m <= kSkinnyMaxRows ? skinny_workspace_bytes(w->type, m, w->n, w->k)
                                            : gemm_workspace_bytes(m, w->n, w->k);

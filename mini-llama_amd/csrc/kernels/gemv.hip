@@ -90,6 +90,7 @@
 #include "../mlq_layout.h"
 #include "device_common.h"
 #include "launch.h"
+#include "weight_decode.h"
 
 namespace mlq {
 namespace {
@@ -159,39 +160,6 @@ __device__ __forceinline__ void load_group(const WaveRsrc& r, Slot<QT>& s,
   if (QT == MLQ_Q4_1) s.m = buf_load8(r.m, soff, (uint32_t)j * kUnitScaleBytes);
 }
 
-// Exact fp16 decode of 8 codes of one quarter-block (MFMA B fragment).
-template <int QT>
-__device__ __forceinline__ h8_t decode8(uint32_t w0, uint32_t w1) {
-  uint4 o;
-  if (QT == MLQ_Q8_0) {
-    const h2_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    uint32_t p0, p1, p2, p3;
-    q8_pairs(w0, p0, p1);
-    q8_pairs(w1, p2, p3);
-    o.x = as_u32(as_h2(p0) - bias);
-    o.y = as_u32(as_h2(p1) - bias);
-    o.z = as_u32(as_h2(p2) - bias);
-    o.w = as_u32(as_h2(p3) - bias);
-  } else {
-    const float lo = QT == MLQ_Q4_0 ? 1032.0f : 1024.0f;
-    const float hi = QT == MLQ_Q4_0 ? 72.0f : 64.0f;
-    const h2_t blo = {(_Float16)lo, (_Float16)lo};
-    const h2_t bhi = {(_Float16)hi, (_Float16)hi};
-    const Q4Pairs p = q4_pairs(w0);
-    o.x = as_u32(as_h2(p.p0) - blo);
-    o.y = as_u32(as_h2(p.p1) - bhi);
-    o.z = as_u32(as_h2(p.p2) - blo);
-    o.w = as_u32(as_h2(p.p3) - bhi);
-  }
-  return __builtin_bit_cast(h8_t, o);
-}
-
-__device__ __forceinline__ _Float16 half_at(uint2 s, int j) {
-  const uint32_t w = (j & 2) ? s.y : s.x;
-  return __builtin_bit_cast(_Float16,
-                            (uint16_t)((j & 1) ? (w >> 16) : (w & 0xffffu)));
-}
-
 // Four activations x[row][4c .. 4c+3] of the slice (zeros past the range).
 // vec: the range is a whole number of float4 (k % 4 == 0); otherwise every
 // element is range-checked on its own.
@@ -203,16 +171,6 @@ __device__ __forceinline__ float4 load_x4(rsrc_t r, int c, bool vec) {
   v.z = __builtin_bit_cast(float, buf_load4(r, (uint32_t)c * 16u + 8u, 0));
   v.w = __builtin_bit_cast(float, buf_load4(r, (uint32_t)c * 16u + 12u, 0));
   return v;
-}
-
-// fp32 pair -> fp16 hi pair + fp16 lo pair with hi + lo = (a, b) to ~2^-22.
-__device__ __forceinline__ void split2(float a, float b, uint32_t& hi,
-                                       uint32_t& lo) {
-  const h2_t h = __builtin_convertvector((f2_t){a, b}, h2_t);
-  const h2_t l = __builtin_convertvector(
-      (f2_t){a - (float)h.x, b - (float)h.y}, h2_t);
-  hi = as_u32(h);
-  lo = as_u32(l);
 }
 
 // hi/lo split of four activations, scaled by 2^e, written at column kl of
@@ -285,12 +243,6 @@ __device__ __forceinline__ int block_sum8_i(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
   v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);  // row_half_mirror
   return v;
-}
-
-// Largest |x| of four activations, NaN propagating (v_maximum3_f32).
-__device__ __forceinline__ float abs_maximum4(float m, float4 v) {
-  m = __builtin_elementwise_maximum(m, __builtin_elementwise_maximum(fabsf(v.x), fabsf(v.y)));
-  return __builtin_elementwise_maximum(m, __builtin_elementwise_maximum(fabsf(v.z), fabsf(v.w)));
 }
 
 // Sum of 8 consecutive lanes' values (one 32-element block = 8 float4):
@@ -1199,6 +1151,7 @@ hipError_t allow_dynamic_lds(const void* kernel, size_t lds) {
 }
 
 void set_gemv_split(int split) { g_split_override = split; }
+bool gemv_split_set() { return g_split_override != 0; }
 
 bool gemv_norm_supported(const mlq_weight& w) {
   if (w.type != MLQ_Q8_0 && w.type != MLQ_Q4_0 && w.type != MLQ_Q4_1) return false;

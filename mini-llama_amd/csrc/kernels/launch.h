@@ -96,6 +96,7 @@ bool gemv_norm_supported(const mlq_weight& w);
 bool gemv_prenorm_supported(const mlq_weight& w);
 // Split override (0 = automatic); validated by the caller.
 void set_gemv_split(int split);
+bool gemv_split_set();
 
 // gemm_mfma.hip: any m >= 1. The _ws form converts x to fp16 into `ws`
 // first when ws_bytes >= f16_copy_bytes(m, k) (else reads fp32 x), and
@@ -143,6 +144,15 @@ hipError_t launch_split_reduce(const float* part, float* y, int m, int n, int sp
                                const Epilogue& epi, hipStream_t stream,
                                const GemmOut& out = GemmOut());
 
+// rows.hip: 2..16 rows of x kept in LDS (k % 4 == 0 and k within its LDS
+// budget, rows_supported), one workgroup per CU streaming its share of the
+// weight tiles; no workspace. rows_faster: the shapes it takes from the
+// decode GEMV and the skinny GEMM.
+bool rows_supported(int type, int m, int n, int k);
+bool rows_faster(int m, int n, int k);
+hipError_t launch_rows(const mlq_weight& w, const float* x, float* y, int m, hipStream_t stream,
+                       const Epilogue& epi = Epilogue());
+
 // skinny.hip: 9..64 rows of x. launch_skinny_ws makes the fragment-ordered
 // fp16 copy of x in ws (not for 9..16 rows with k <= 6144, k % 4 == 0:
 // that kernel reads fp32 x itself), then runs the skinny GEMM (K split over
@@ -158,6 +168,7 @@ hipError_t launch_skinny_ws(const mlq_weight& w, const float* x, float* y, int m
 // Plan override (0 = planner): weight tiles per workgroup (1, 2, 4) and K
 // ranges per tile group (1..8); validated by the caller.
 void set_skinny_plan(int tiles, int splits);
+bool skinny_plan_set();
 
 // aos_gemv.hip: GEMV straight from GGUF AoS blocks (m <= 8 rows of x, x
 // staged in LDS: aos_gemv_supported says whether the shape fits).

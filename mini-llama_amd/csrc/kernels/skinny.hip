@@ -52,6 +52,7 @@
 #include "device_common.h"
 #include "launch.h"
 #include "row_copy.h"
+#include "weight_decode.h"
 
 namespace mlq {
 namespace {
@@ -107,51 +108,10 @@ __device__ __forceinline__ void load_group(Group<QT, MB, T>& gr, const rsrc_t (&
       gr.a[mb][b] = buf_load16(rx, (uint32_t)((((j * MB + mb) * 4 + b) * 64 + lane) * 16), 0);
 }
 
-__device__ __forceinline__ h2_t splat(uint2 s, int b) {
-  const uint32_t w = (b & 2) ? s.y : s.x;
-  const _Float16 v = __builtin_bit_cast(_Float16, (uint16_t)((b & 1) ? (w >> 16) : (w & 0xffffu)));
-  return (h2_t){v, v};
-}
-
-// B fragment of block b of tile t: 8 codes of quarter lane/16 of row
-// lane%16, decoded exactly and scaled in fp16.
+// B fragment of block b of tile t: 8 codes of quarter lane/16 of row lane%16.
 template <int QT, int MB, int T>
 __device__ __forceinline__ h8_t decode(const Group<QT, MB, T>& gr, int t, int b) {
-  const h2_t d2 = splat(gr.d[t], b);
-  uint4 o;
-  if (QT == MLQ_Q8_0) {
-    const uint4 q = b < 2 ? gr.q[t] : gr.q2[t];
-    const uint32_t w0 = (b & 1) ? q.z : q.x, w1 = (b & 1) ? q.w : q.y;
-    const h2_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    uint32_t p0, p1, p2, p3;
-    q8_pairs(w0, p0, p1);
-    q8_pairs(w1, p2, p3);
-    o.x = as_u32((as_h2(p0) - bias) * d2);
-    o.y = as_u32((as_h2(p1) - bias) * d2);
-    o.z = as_u32((as_h2(p2) - bias) * d2);
-    o.w = as_u32((as_h2(p3) - bias) * d2);
-  } else {
-    const uint4 qq = gr.q[t];
-    const uint32_t w = b == 0 ? qq.x : b == 1 ? qq.y : b == 2 ? qq.z : qq.w;
-    const float lo = QT == MLQ_Q4_0 ? 1032.0f : 1024.0f;
-    const float hi = QT == MLQ_Q4_0 ? 72.0f : 64.0f;
-    const h2_t blo = {(_Float16)lo, (_Float16)lo};
-    const h2_t bhi = {(_Float16)hi, (_Float16)hi};
-    const Q4Pairs p = q4_pairs(w);
-    if (QT == MLQ_Q4_0) {
-      o.x = as_u32((as_h2(p.p0) - blo) * d2);
-      o.y = as_u32((as_h2(p.p1) - bhi) * d2);
-      o.z = as_u32((as_h2(p.p2) - blo) * d2);
-      o.w = as_u32((as_h2(p.p3) - bhi) * d2);
-    } else {
-      const h2_t m2 = splat(gr.mm[t], b);
-      o.x = as_u32(__builtin_elementwise_fma(as_h2(p.p0) - blo, d2, m2));
-      o.y = as_u32(__builtin_elementwise_fma(as_h2(p.p1) - bhi, d2, m2));
-      o.z = as_u32(__builtin_elementwise_fma(as_h2(p.p2) - blo, d2, m2));
-      o.w = as_u32(__builtin_elementwise_fma(as_h2(p.p3) - bhi, d2, m2));
-    }
-  }
-  return __builtin_bit_cast(h8_t, o);
+  return decode_scaled<QT>(gr.q[t], gr.q2[t], gr.d[t], gr.mm[t], b);
 }
 
 // Groups a wave keeps in flight: as many as ~160 registers less the
@@ -360,18 +320,10 @@ __device__ __forceinline__ void load_lines2(Lines2<QT, T>& w, const rsrc_t (&rq)
   }
 }
 
-// B fragment of block b of group gi, tile t (decode() of a Group).
+// B fragment of block b of group gi, tile t.
 template <int QT, int T>
 __device__ __forceinline__ h8_t decode2(const Lines2<QT, T>& w, int gi, int t, int b) {
-  Group<QT, 1, T> g1;
-#pragma unroll
-  for (int u = 0; u < T; ++u) {
-    g1.q[u] = w.q[gi][u];
-    g1.q2[u] = w.q2[gi][u];
-    g1.d[u] = w.d[gi][u];
-    g1.mm[u] = w.mm[gi][u];
-  }
-  return decode<QT, 1, T>(g1, t, b);
+  return decode_scaled<QT>(w.q[gi][t], w.q2[gi][t], w.d[gi][t], w.mm[gi][t], b);
 }
 
 // Largest of a non-negative value over the four lanes of a quad (every lane
@@ -381,15 +333,6 @@ __device__ __forceinline__ float quad_max_nonneg(float v) {
   b = max(b, __builtin_amdgcn_mov_dpp(b, 0xB1, 0xF, 0xF, false));  // quad_perm [1,0,3,2]
   b = max(b, __builtin_amdgcn_mov_dpp(b, 0x4E, 0xF, 0xF, false));  // quad_perm [2,3,0,1]
   return __builtin_bit_cast(float, b);
-}
-
-// Largest |x| of four values joined to m; NaN propagates (a NaN row's
-// output is NaN whatever its scale). Two v_maximum3_f32 with abs modifiers.
-__device__ __forceinline__ float abs_maximum4(float m, float4 v) {
-  m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(v.x)),
-                                    __builtin_fabsf(v.y));
-  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(v.z)),
-                                       __builtin_fabsf(v.w));
 }
 
 // x * 2^e rounded once to fp16 (v_fma_mixlo / mixhi: the scaling is exact,
@@ -687,6 +630,7 @@ void set_skinny_plan(int tiles, int splits) {
   g_tiles_override = tiles;
   g_splits_override = splits;
 }
+bool skinny_plan_set() { return g_tiles_override != 0 || g_splits_override != 0; }
 
 // fp16 copy path: x copy, its row exponents (one per padded row), then
 // (split K) the partial slices; fp32-input kernel: the partial slices only.

@@ -746,3 +746,37 @@ def test_cpp_interface_tests(pkg):
     print(r.stderr[-4000:])
     assert r.returncode == 0
     assert "(skip" not in r.stdout
+
+
+# ---- 2..16 rows with x resident in LDS (rows.hip) ---------------------------------------------------
+# 5..16 rows from 321 weight tiles on, 2..4 rows from 32768 units on, and rows too long for the GEMV's
+# staging: runs of units shorter than a tile, whole tiles inside a run, uneven tile counts, the longest
+# K of each row count, ragged K and N, the padded row counts' edges.
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("m,n,k", [(5, 5137, 100), (8, 5136, 132), (9, 5152, 36), (16, 5121, 4100), (12, 8208, 4864),
+                                   (8, 9001, 4736), (16, 40000, 256), (2, 8209, 8196), (3, 16401, 4096),
+                                   (4, 16400, 4228), (2, 3584, 17408), (3, 640, 9216), (6, 100, 4864)])
+def test_resident_rows(pkg, cuda, qtype, m, n, k):
+    import torch
+    from synthetic import synth
+    _print_case(test="resident_rows", qtype=qtype, m=m, n=n, k=k)
+    g = torch.Generator(device=cuda).manual_seed(m + n + k)
+    tw = pkg.repack_device(qtype, synth.device_blocks(torch, g, qtype, n, k, 0.02, cuda).view(-1).view(torch.uint8), n, k)
+    x = torch.randn((m, k), generator=g, device=cuda)
+    x[0] *= 1e12
+    x[m - 1] *= 1e-12
+    bias = torch.randn(n, generator=g, device=cuda)
+    w64, x64 = pkg.dequantize(tw).double(), x.double()
+    ref = x64 @ w64.t().contiguous() + bias.double()
+    size = x64.abs() @ w64.abs().t().contiguous() + bias.abs().double()
+    # up to 8 rows (where the longest x fits): x to 2^-22, fp32 sums; more: x and W rounded to fp16 once
+    grow = 2.0 ** -20 if m <= 8 and pkg.workspace_bytes(tw, m) == 0 else 2.0 ** -10
+    y = pkg.linear(tw, x, bias=bias).double()
+    assert bool(((y - ref).abs() <= grow * size).all())
+    if n % 16 == 0:
+        t, e = ref.view(m, n // 16, 2, 8), (grow * size).view(m, n // 16, 2, 8)
+        gate, up = t[:, :, 0], t[:, :, 1]
+        y = pkg.linear(tw, x, bias=bias, act=pkg.EPI_SWIGLU).double().view(m, n // 16, 8)
+        slack = 1.1 * e[:, :, 0] * (up.abs() + e[:, :, 1]) + gate.abs() * e[:, :, 1]
+        slack = slack + 16 * 2.0 ** -23 * (gate * up).abs() + 1e-30
+        assert bool(((y - torch.nn.functional.silu(gate) * up).abs() <= slack).all())
