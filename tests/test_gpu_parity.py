@@ -780,3 +780,25 @@ def test_resident_rows(pkg, cuda, qtype, m, n, k):
         slack = 1.1 * e[:, :, 0] * (up.abs() + e[:, :, 1]) + gate.abs() * e[:, :, 1]
         slack = slack + 16 * 2.0 ** -23 * (gate * up).abs() + 1e-30
         assert bool(((y - torch.nn.functional.silu(gate) * up).abs() <= slack).all())
+
+
+# Raw GGUF blocks with several tiles per workgroup (whole and shared ones), odd block counts (rows off
+# 4-byte boundaries), k % 4 != 0, a base off a 4-byte boundary, blocks of the last group past the row.
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("m,n,k", [(1, 9001, 1056), (3, 8200, 3104), (8, 4500, 994), (1, 20000, 99), (2, 16411, 128)])
+def test_aos_many_tiles(pkg, cuda, qtype, m, n, k):
+    import torch
+    from synthetic import synth
+    _print_case(test="aos_many_tiles", qtype=qtype, m=m, n=n, k=k)
+    g = torch.Generator(device=cuda).manual_seed(m + n + k)
+    raw = synth.device_blocks(torch, g, qtype, n, k, 0.02, cuda).view(-1).view(torch.uint8)
+    x = torch.randn((m, k), generator=g, device=cuda)
+    w64, x64 = pkg.dequantize(pkg.repack_device(qtype, raw, n, k)).double(), x.double()
+    ref = x64 @ w64.t().contiguous()
+    # x to 2^-22, fp32 sums
+    bound = 2.0 ** -20 * (x64.abs() @ w64.abs().t().contiguous())
+    for lead in (0, 2):
+        buf = torch.zeros(raw.numel() + 16, dtype=torch.uint8, device=cuda)
+        buf[lead:lead + raw.numel()] = raw
+        y = pkg.linear_aos(qtype, buf[lead:lead + raw.numel()], n, k, x).view(m, n).double()
+        assert bool(((y - ref).abs() <= bound).all()), lead
