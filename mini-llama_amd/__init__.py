@@ -231,9 +231,11 @@ def repack_host(qtype: str, blocks: np.ndarray, n: int, k: int):
 
 
 def _stream(stream=None) -> int:
+    if stream is not None:
+        return stream.cuda_stream
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    # the handle alone: building a Stream object takes 3 us, as long as a launch
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 class TiledWeight:
@@ -491,17 +493,20 @@ def linear(w: TiledWeight, x, y=None, path: int = PATH_AUTO, stream=None,
         shape = (ny,) if x.dim() == 1 else (m, ny)
         y = torch.empty(shape, dtype=torch.float32, device=x.device)
     if path == PATH_AUTO and workspace is not None:
-        need = workspace_bytes(w, m)
-        ws = workspace
-        if isinstance(workspace, str):
-            ws = _workspace(x.device, need) if need else None
-        ws_ptr = ws.data_ptr() if ws is not None else None
-        ws_len = ws.numel() * ws.element_size() if ws is not None else 0
-        _check(lib().mlq_linear_epi(ctypes.byref(w.layout), x.data_ptr(),
-                                    y.data_ptr(), m,
-                                    bias.data_ptr() if bias is not None else None,
-                                    act, ws_ptr, ws_len, _stream(stream)),
-               "mlq_linear_epi")
+        auto = isinstance(workspace, str)
+        ws = _WORKSPACES.get(x.device.index or 0) if auto else workspace
+        layout, bp = ctypes.byref(w.layout), bias.data_ptr() if bias is not None else None
+
+        def call():
+            return lib().mlq_linear_epi(
+                layout, x.data_ptr(), y.data_ptr(), m, bp, act,
+                ws.data_ptr() if ws is not None else None,
+                ws.numel() * ws.element_size() if ws is not None else 0, _stream(stream))
+        status = call()
+        if status == -4 and auto:  # nothing ran: the workspace has to grow
+            ws = _workspace(x.device, workspace_bytes(w, m))
+            status = call()
+        _check(status, "mlq_linear_epi")
         return y
     _check(lib().mlq_linear_path(ctypes.byref(w.layout), x.data_ptr(),
                                  y.data_ptr(), m, path, _stream(stream)),

@@ -81,6 +81,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 #include <mutex>
 #include <set>
@@ -1151,7 +1152,7 @@ hipError_t allow_dynamic_lds(const void* kernel, size_t lds) {
 }
 
 void set_gemv_split(int split) { g_split_override = split; }
-bool gemv_split_set() { return g_split_override != 0; }
+bool gemv_split_set() { return split_override() != 0; }
 
 bool gemv_norm_supported(const mlq_weight& w) {
   if (w.type != MLQ_Q8_0 && w.type != MLQ_Q4_0 && w.type != MLQ_Q4_1) return false;
@@ -1173,7 +1174,20 @@ bool gemv_prenorm_supported(const mlq_weight& w) {
 }
 
 int gemv_max_k(int type, int m) {
-  if (m < 1 || m > kGemvMaxRows) return 0;
+  if (m < 1 || m > kGemvMaxRows || type < MLQ_Q8_0 || type > MLQ_Q4_1) return 0;
+  // Every Linear call asks; the search plans up to 300 lengths (4 us), so its
+  // answers are kept per type, rows and split override (log2; 0 = none).
+  static std::atomic<int> known[6][3][kGemvMaxRows];
+  const int split = split_override();
+  int slot = 0;
+  while (slot < 5 && split != 0 && split != 1 << slot) ++slot;
+  slot = split == 0 ? 5 : slot;  // (an environment value that is no power of two: 5 too)
+  const bool keep = split == 0 || (slot < 5 && split == 1 << slot);
+  std::atomic<int>& answer = known[slot][type - MLQ_Q8_0][m - 1];
+  if (keep) {
+    const int k = answer.load(std::memory_order_relaxed);
+    if (k != 0) return k - 1;
+  }
   // the largest K whose default plan fits the LDS budget
   int best = 0;
   for (int g = 1; g <= 4096; ++g) {
@@ -1181,6 +1195,7 @@ int gemv_max_k(int type, int m) {
     if (make_plan(type, m, geo).lds > lds_limit()) break;
     best = g * kGroupK;
   }
+  if (keep) answer.store(best + 1, std::memory_order_relaxed);
   return best;
 }
 
