@@ -1014,6 +1014,247 @@ __global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(At
   }
 }
 
+// ---- prefill attention, many rows: fp16 pairs on v_mfma_f32_32x32x16_f16 ---------------
+// The kernel above is bound by the fp32 matrix rate (57 TFLOP/s of the causal
+// products at 2000 tokens, 28 heads on 4: 498 us, this one 182). Here
+// every operand is split into two fp16 values, x = hi + lo to 2^-23 of x (its
+// row first scaled by a power of two into fp16's range), and a product is
+// hi hi + hi lo + lo hi (the dropped lo lo is below 2^-24 of it): three
+// products at sixteen times the rate.
+//  - A workgroup owns 128 (query row, head) pairs of one kv head, a wave 32 of
+//    them as the columns of both products, S^T = K Q^T and O^T = V^T P^T. A
+//    lane then holds 16 keys of one column, so the softmax over keys is in
+//    registers but for one lane swap, and P^T is already the B operand of the
+//    second product: its k slots take the keys in the order the first one
+//    leaves them, and V^T is stored in that order.
+//  - Tiles of 32 keys: each thread splits 4 keys x 4 dims of K and of V into
+//    LDS (V transposed in registers), double buffered, the next tile's rows
+//    in flight; one barrier per tile.
+//  - Scales: K per four keys (applied to the scores), Q per row, V per four keys, folded
+//    into P relative to the largest seen (the accumulators are rescaled when
+//    that grows); P itself is kept times 2^14, so its low half stays above
+//    fp16's subnormals.
+//  - Workgroups with the most keys start first; the kv head is the fastest
+//    grid index, so with 4 or 8 of them an XCD's L2 serves one or two.
+constexpr int kPairRows = 128, kPairKeys = 32;
+template <int HD>
+struct PairTile {
+  _Float16 k[2][kPairKeys][HD + 8];   // hi, lo: [key][dim]
+  _Float16 v[2][HD][kPairKeys + 8];   // hi, lo: [dim][key slot], see v_unit
+  float ks[kPairKeys / 4], vs[kPairKeys / 4];  // 2^-e of four keys' K and V
+};
+
+// Where the 8-slot unit of a dim's row lies: a thread writes four dims of four
+// keys, so neighbouring lanes are four rows (16 banks) apart; turning the
+// units by the dim spreads 16 of them over the banks.
+__device__ __forceinline__ int v_unit(int unit, int dim) { return (unit ^ ((dim >> 4) & 3)) * 8; }
+__device__ __forceinline__ uint2 pack4(_Float16 a, _Float16 b, _Float16 c, _Float16 d) {
+  return make_uint2(as_u32(h2_t{a, b}), as_u32(h2_t{c, d}));
+}
+
+template <int HD, int GP>
+__global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
+  constexpr int KT = HD / 16;   // 16-dim steps of the scores
+  constexpr int VB = HD / 32;   // 32-dim blocks of the output
+  constexpr int DG = HD / 4;    // threads across a key's dims
+  extern __shared__ __align__(16) uint8_t pair_smem[];
+  PairTile<HD>* tiles = (PairTile<HD>*)pair_smem;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, half = lane >> 5;
+  const int G = a.group;
+  const int kvh = blockIdx.x % a.n_kv;
+  const int r0 = ((int)(gridDim.x / a.n_kv) - 1 - (int)(blockIdx.x / a.n_kv)) * (kPairRows / GP);
+  const int kmax = a.pos + min(r0 + kPairRows / GP, a.rows) - 1;  // last key any row sees
+  const int nt = kmax / kPairKeys + 1;
+  const size_t row_stride = (size_t)a.n_kv * HD;
+  const size_t cbase = (size_t)a.layer * a.max_seq * row_stride + (size_t)kvh * HD;
+  const uint32_t rs4 = (uint32_t)row_stride * 4u;
+  const uint32_t kvbytes = (uint32_t)kmax * rs4 + HD * 4u;  // rows past kmax read as zeros
+  const rsrc_t rk = make_rsrc(a.keys + cbase, kvbytes);
+  const rsrc_t rv = make_rsrc(a.values + cbase, kvbytes);
+
+  // this thread's piece of a tile: keys 4 kg .. + 3, dims 4 dg .. + 3
+  const int dg = tid % DG, kg = tid / DG;
+  const bool loads = kg < kPairKeys / 4;  // (HD 64: half of the threads)
+  f4_t kr[4], vr[4];
+  auto load = [&](int t) __attribute__((always_inline)) {
+    const uint32_t off = loads ? (uint32_t)(t * kPairKeys + 4 * kg) * rs4 + 16u * dg : 0x80000000u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      kr[i] = __builtin_bit_cast(f4_t, buf_load16(rk, off + i * rs4, 0));
+      vr[i] = __builtin_bit_cast(f4_t, buf_load16(rv, off + i * rs4, 0));
+    }
+  };
+  auto amax = [&](const f4_t (&r)[4]) __attribute__((always_inline)) {
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      mx = fmaxf(fmaxf(fmaxf(mx, fabsf(r[i].x)), fmaxf(fabsf(r[i].y), fabsf(r[i].z))), fabsf(r[i].w));
+    return row_max<DG>(mx);
+  };
+  auto split = [&](PairTile<HD>& t) __attribute__((always_inline)) {
+    // slot of the key group in a 16-key run: keys 0-3, 8-11 | 4-7, 12-15
+    const int unit = 2 * (kg >> 2) + (kg & 1), sub = 4 * ((kg >> 1) & 1);
+    const float ka = amax(kr), va = amax(vr);
+    const int ke = min(pow2_scale_exp(ka), 126), ve = min(pow2_scale_exp(va), 126);
+    const float kf = ldexp_f(1.0f, ke), vf = ldexp_f(1.0f, ve);
+    if (!loads) return;
+    if (dg == 0) {
+      t.ks[kg] = ldexp_f(1.0f, -ke);
+      t.vs[kg] = va == 0.0f ? 0.0f : ldexp_f(1.0f, -ve);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      _Float16 h[4], l[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float x = kr[i][j] * kf;
+        h[j] = (_Float16)x;
+        l[j] = (_Float16)(x - (float)h[j]);
+      }
+      *(uint2*)&t.k[0][4 * kg + i][4 * dg] = pack4(h[0], h[1], h[2], h[3]);
+      *(uint2*)&t.k[1][4 * kg + i][4 * dg] = pack4(l[0], l[1], l[2], l[3]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // dim 4 dg + j of the four keys
+      _Float16 h[4], l[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float y = vr[i][j] * vf;
+        h[i] = (_Float16)y;
+        l[i] = (_Float16)(y - (float)h[i]);
+      }
+      const int dim = 4 * dg + j, at = v_unit(unit, dim) + sub;
+      *(uint2*)&t.v[0][dim][at] = pack4(h[0], h[1], h[2], h[3]);
+      *(uint2*)&t.v[1][dim][at] = pack4(l[0], l[1], l[2], l[3]);
+    }
+  };
+
+  // this lane's column: query row qr, head qh of the group
+  const int c0 = wave * 32;
+  const int qr = r0 + (c0 + col) / GP, qh = (c0 + col) % GP;
+  const bool live = qr < a.rows && qh < G;
+  const int qpos = a.pos + qr;
+  const int wmin = a.pos + r0 + c0 / GP;  // the first and last key the wave's rows see
+  const int wmax = min(a.pos + r0 + (c0 + 31) / GP, kmax);
+  h8_t qhi[KT], qlo[KT];
+  float qscale;
+  {
+    const float* qp = a.q + (size_t)(live ? qr : 0) * a.q_stride +
+                      (size_t)(kvh * G + (live ? qh : 0)) * HD + 8 * half;
+    f4_t x[KT][2];
+    float mx = 0.0f;
+#pragma unroll
+    for (int s = 0; s < KT; ++s)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        x[s][u] = live ? *(const f4_t*)(qp + 16 * s + 4 * u) : f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, fabsf(x[s][u][j]));
+      }
+    const int e = min(pow2_scale_exp(xor32_max(mx)), 126);
+    const float f = ldexp_f(1.0f, e);
+    // softmax in base 2: scores times scale log2(e)
+    qscale = a.scale * 1.44269504088896341f * ldexp_f(1.0f, -e);
+#pragma unroll
+    for (int s = 0; s < KT; ++s)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = x[s][j >> 2][j & 3] * f;
+        qhi[s][j] = (_Float16)v;
+        qlo[s][j] = (_Float16)(v - (float)qhi[s][j]);
+      }
+  }
+
+  typedef float f16v __attribute__((ext_vector_type(16)));
+  f16v acc[VB];
+#pragma unroll
+  for (int b = 0; b < VB; ++b) acc[b] = (f16v){};
+  float m = -INFINITY, l = 0.0f;  // of the column; l of this half's keys
+  float ref = 0.0f;               // largest V scale so far (wave-uniform)
+
+  load(0);
+  for (int t = 0; t < nt; ++t) {
+    PairTile<HD>& tl = tiles[t & 1];
+    split(tl);
+    if (t + 1 < nt) load(t + 1);
+    __syncthreads();
+    const int k0 = t * kPairKeys;
+    if (k0 > wmax) continue;  // (the wave's rows end before this tile)
+    f16v s = {};
+#pragma unroll
+    for (int i = 0; i < KT; ++i) {
+      const h8_t kh = *(const h8_t*)&tl.k[0][col][16 * i + 8 * half];
+      const h8_t kl = *(const h8_t*)&tl.k[1][col][16 * i + 8 * half];
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qhi[i], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qlo[i], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qhi[i], s, 0, 0, 0);
+    }
+    // lane: keys 8 (i / 4) + 4 half + i % 4 of its column
+    float vsc[4], mx = m, vmax = ref;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float ks = tl.ks[2 * q + half] * qscale;
+      vsc[q] = tl.vs[2 * q + half];
+      vmax = fmaxf(vmax, vsc[q]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[4 * q + j] *= ks;
+    }
+    if (k0 + kPairKeys - 1 > wmin) {  // the causal edge crosses the tile
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        s[i] = k0 + 8 * (i >> 2) + 4 * half + (i & 3) <= qpos ? s[i] : -INFINITY;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    mx = xor32_max(mx);
+    vmax = xor32_max(vmax);
+    // rows with nothing visible yet keep m = -inf and weight 0
+    const float base = mx == -INFINITY ? 0.0f : mx;
+    const float alpha = mx == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mx);
+    const float inv = vmax > 0.0f ? 1.0f / vmax : 0.0f;  // powers of two
+    if (__any(alpha != 1.0f) || vmax != ref) {
+      const float f = alpha * (ref * inv);
+#pragma unroll
+      for (int b = 0; b < VB; ++b) acc[b] *= f;
+      l *= alpha;
+    }
+    m = mx;
+    ref = vmax;
+    h8_t ph[2], pl[2];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float p = __builtin_amdgcn_exp2f(s[i] - base + 14.0f);
+      l += p;
+      const float w = p * (vsc[i >> 2] * inv);
+      const _Float16 h = (_Float16)w;
+      ph[i >> 3][i & 7] = h;
+      pl[i >> 3][i & 7] = (_Float16)(w - (float)h);
+    }
+#pragma unroll
+    for (int b = 0; b < VB; ++b)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int at = v_unit(2 * u + half, 32 * b + col);
+        const h8_t vh = *(const h8_t*)&tl.v[0][32 * b + col][at];
+        const h8_t vl = *(const h8_t*)&tl.v[1][32 * b + col][at];
+        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph[u], acc[b], 0, 0, 0);
+        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[u], acc[b], 0, 0, 0);
+        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[u], acc[b], 0, 0, 0);
+      }
+  }
+  if (!live) return;
+  const float f = ref / xor32_sum(l);
+  float* out = a.out + (size_t)qr * a.out_stride + (size_t)(kvh * G + qh) * HD;
+#pragma unroll
+  for (int b = 0; b < VB; ++b)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *(f4_t*)(out + 32 * b + 8 * q + 4 * half) =
+          f4_t{acc[b][4 * q] * f, acc[b][4 * q + 1] * f, acc[b][4 * q + 2] * f, acc[b][4 * q + 3] * f};
+}
+
 // e^(s - m) for s <= m as 2^h (1 + f ln 2), h + f = (s - m) log2 e with h the
 // rounded product and f what it lost (log2 e in two parts): the hardware
 // exp2's own error and no more.
@@ -1914,20 +2155,37 @@ bool prefill_attention_supported(int hd, int group) {
 }
 
 template <int HD, int GP>
-static void prefill_launch(const AttnArgs& a, hipStream_t stream) {
+static hipError_t prefill_launch(const AttnArgs& a, hipStream_t stream) {
+  if constexpr (HD <= 128) {
+    // 128-row workgroups once they cover 3/8 of the CUs (2 layers of hidden
+    // 3584, FFN 9472, 28 heads on 4: 400 tokens, 100 workgroups, 532 -> 521
+    // us; 600 670 -> 630; 1000 1152 -> 995; 256 tokens, 64 workgroups, 360 ->
+    // 365, so those keep the 16-row tiles)
+    const int groups = (a.rows * GP + kPairRows - 1) / kPairRows * a.n_kv;
+    if (8 * groups >= 3 * device_cus() &&
+        (uint64_t)a.max_seq * a.n_kv * HD * 4 < (1ull << 31)) {  // 31-bit offsets
+      const auto kernel = attn_pair_kernel<HD, GP>;
+      const size_t lds = 2 * sizeof(PairTile<HD>);
+      const hipError_t e = allow_dynamic_lds((const void*)kernel, lds);
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(kernel, dim3(groups), dim3(256), lds, stream, a);
+      return hipGetLastError();
+    }
+  }
   constexpr int QT = 16 / GP;
   const int tiles = (a.rows + QT - 1) / QT;
   hipLaunchKernelGGL((attn_prefill_kernel<HD, GP>), dim3(tiles, a.n_kv),
                      dim3(prefill_waves(HD) * 64), 0, stream, a);
+  return hipGetLastError();
 }
 
 template <int HD>
-static void prefill_launch_g(const AttnArgs& a, hipStream_t stream) {
-  if (a.group <= 1) prefill_launch<HD, 1>(a, stream);
-  else if (a.group <= 2) prefill_launch<HD, 2>(a, stream);
-  else if (a.group <= 4) prefill_launch<HD, 4>(a, stream);
-  else if (a.group <= 8) prefill_launch<HD, 8>(a, stream);
-  else prefill_launch<HD, 16>(a, stream);
+static hipError_t prefill_launch_g(const AttnArgs& a, hipStream_t stream) {
+  if (a.group <= 1) return prefill_launch<HD, 1>(a, stream);
+  if (a.group <= 2) return prefill_launch<HD, 2>(a, stream);
+  if (a.group <= 4) return prefill_launch<HD, 4>(a, stream);
+  if (a.group <= 8) return prefill_launch<HD, 8>(a, stream);
+  return prefill_launch<HD, 16>(a, stream);
 }
 
 hipError_t launch_attention_prefill(const AttnLaunch& r, hipStream_t stream) {
@@ -1952,11 +2210,10 @@ hipError_t launch_attention_prefill(const AttnLaunch& r, hipStream_t stream) {
   // the kernel addresses one layer's K / V rows with 32-bit byte offsets
   if ((uint64_t)r.max_seq * r.n_kv * r.hd * 4 >= (1ull << 32)) return hipErrorInvalidValue;
   switch (r.hd) {
-    case 64: prefill_launch_g<64>(a, stream); break;
-    case 128: prefill_launch_g<128>(a, stream); break;
-    default: prefill_launch_g<256>(a, stream); break;
+    case 64: return prefill_launch_g<64>(a, stream);
+    case 128: return prefill_launch_g<128>(a, stream);
+    default: return prefill_launch_g<256>(a, stream);
   }
-  return hipGetLastError();
 }
 
 hipError_t launch_argmax(const float* x, int64_t n, int32_t* out, int32_t* pos_dev,

@@ -788,6 +788,36 @@ def test_prefill_qwen2_7b_layer_at_full_size(pkg, oracle, cuda, qtype):
     assert np.abs(got - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-6
 
 
+# Long prompts whose 128-row attention workgroups cover 3/8 of the CUs run on fp16 pairs; the same
+# prompt in shorter pieces keeps the fp32 MFMA tiles. Ragged lengths, a past that begins inside a tile
+# and whose values span twelve decades, groups padded from 1, 3, 7 and 12 heads.
+@pytest.mark.parametrize("hd,n_heads,n_kv,n,start", [(128, 28, 4, 413, 70), (64, 8, 8, 1545, 0), (128, 24, 2, 801, 33),
+                                                     (64, 12, 4, 1001, 5), (128, 4, 4, 3100, 1)])
+def test_prefill_long_prompt_pair_attention(pkg, cuda, hd, n_heads, n_kv, n, start):
+    import mini_llama_amd.decode as dec
+    from synthetic import synth
+    import torch
+    cfg = dict(vocab_size=300, dim=128, hidden_dim=64, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv, head_dim=hd,
+               max_seq_len=3200, rope_type=1)
+    dm = dec.DecodeModel(synth.synthetic_model(cfg, "f32", seed=6))
+    g = torch.Generator(device=cuda).manual_seed(n)
+    tokens = np.random.default_rng(n).integers(0, 300, n)
+    past = (dm.keys.shape[0], start, n_kv, hd)
+    k0 = torch.randn(past, generator=g, device=cuda)
+    v0 = torch.randn(past, generator=g, device=cuda) * 10.0 ** torch.randint(-9, 3, past[:3] + (1,), generator=g, device=cuda)
+
+    def run(piece):
+        dm.reset()
+        dm.keys[:, :start], dm.values[:, :start] = k0, v0
+        for lo in range(0, n, piece):
+            logits = dm.prefill(tokens[lo:lo + piece], start + lo)
+        return logits.clone(), dm.keys.clone(), dm.values.clone()
+
+    whole, pieces = run(n), run(180)
+    for a, b in zip(whole, pieces):  # fp32 Linears both times: only sums in other orders
+        assert float((a - b).abs().max()) <= 3e-5 * float(b.abs().max())
+
+
 def test_prefill_tiny_model_greedy(pkg, oracle, cuda):
     """The reference's tiny model (F32 weights): greedy generation with the
     prompt prefilled in one batch picks the oracle's tokens."""
