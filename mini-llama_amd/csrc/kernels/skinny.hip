@@ -47,6 +47,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "../mlq_layout.h"
 #include "device_common.h"
@@ -276,6 +277,158 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(SkinnyArgs a) {
   finish<T, MB>(a, acc, part, sp, t0);
 }
 
+// ---- many weight tiles: x shared through LDS ---------------------------------
+// With more tiles than the chip takes at once, a workgroup per T tiles reads
+// the x of its K range once per T tiles (64 rows of 37888 x 3584: 272 MB from
+// L2 for 76 MB of weights) and holds so many registers that only one group of
+// it is in flight: 45 us where the weights take 12. Here one workgroup per CU
+// owns nt / CUs tiles, a wave one or two of them over all of K (no slices to
+// combine), and the x fragments of 256 k at a time pass through LDS to all
+// eight waves: x crosses to a CU once. Two stages of x and the next stage's
+// weight lines are in registers, two LDS slabs, one barrier per stage.
+constexpr int kWideGroups = 2;  // 128-k groups per stage
+
+template <int QT, int MB>
+struct WideLines {
+  uint4 q[kWideGroups], q2[kWideGroups];
+  uint2 d[kWideGroups], mm[kWideGroups];
+};
+
+template <int QT, int MB>
+__global__ __launch_bounds__(kThreads) void skinny_wide_kernel(SkinnyArgs a) {
+  constexpr int kGroupBytes = MB * 4096;
+  constexpr int kStage = kWideGroups * kGroupBytes;
+  constexpr int kLoads = kStage / (16 * kThreads);  // 16-byte pieces per thread
+  static_assert(kLoads * 16 * kThreads == kStage, "a stage is whole loads");
+  __shared__ __attribute__((aligned(16))) uint8_t slab[2][kStage];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grid = gridDim.x;
+  const int each = a.nt / grid, extra = a.nt % grid;
+  const int T = each + ((int)blockIdx.x < extra ? 1 : 0);
+  const int t0 = (int)blockIdx.x * each + min((int)blockIdx.x, extra);
+  const int stages = (a.g + kWideGroups - 1) / kWideGroups;
+  constexpr uint32_t QB = QT == MLQ_Q8_0 ? 2048u : 1024u;
+  const rsrc_t rx = make_rsrc(a.xf, (uint32_t)a.g * kGroupBytes);
+  using Lines = WideLines<QT, MB>;
+
+  for (int p0 = 0; p0 < T; p0 += 2 * kWaves) {  // sixteen tiles at a time
+    const int n = min(T - p0, 2 * kWaves);
+    // this wave's tiles wave and wave + 8 of the pass (past it: zeros)
+    rsrc_t rq[2], rd[2], rm[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int at = wave + kWaves * t;
+      const size_t unit0 = (size_t)(t0 + p0 + min(at, n - 1)) * a.g;
+      const uint32_t units = at < n ? (uint32_t)a.g : 0u;
+      rq[t] = make_rsrc(a.qs + unit0 * QB, units * QB);
+      rd[t] = make_rsrc(a.d + unit0 * 128, units * 128u);
+      rm[t] = QT == MLQ_Q4_1 ? make_rsrc(a.mn + unit0 * 128, units * 128u) : rd[t];
+    }
+    auto load_w = [&](Lines& w, int t, int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int g = 0; g < kWideGroups; ++g) {
+        const uint32_t unit = (uint32_t)(s * kWideGroups + g);
+        w.q[g] = buf_load16_stream(rq[t], (uint32_t)lane * 16u, unit * QB);
+        if (QT == MLQ_Q8_0) w.q2[g] = buf_load16_stream(rq[t], (uint32_t)lane * 16u, unit * QB + 1024u);
+        w.d[g] = buf_load8(rd[t], (uint32_t)(lane & 15) * 8u, unit * 128u);
+        if (QT == MLQ_Q4_1) w.mm[g] = buf_load8(rm[t], (uint32_t)(lane & 15) * 8u, unit * 128u);
+      }
+    };
+    uint4 even[kLoads], odd[kLoads];
+    auto load_x = [&](uint4 (&v)[kLoads], int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        v[i] = buf_load16(rx, (uint32_t)(tid + i * kThreads) * 16u, (uint32_t)s * kStage);
+    };
+    auto store_x = [&](const uint4 (&v)[kLoads], int buf) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) *(uint4*)(slab[buf] + (tid + i * kThreads) * 16) = v[i];
+    };
+    f4_t acc[2][MB];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) acc[t][mb] = (f4_t){0.f, 0.f, 0.f, 0.f};
+    const bool two = wave + kWaves < n;
+    auto run = [&](const Lines (&w)[2], int buf, auto both) __attribute__((always_inline)) {
+      constexpr int NT = decltype(both)::value ? 2 : 1;
+#pragma unroll
+      for (int g = 0; g < kWideGroups; ++g)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          h8_t bf[NT];
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            bf[t] = decode_scaled<QT>(w[t].q[g], w[t].q2[g], w[t].d[g], w[t].mm[g], b);
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) {
+            const h8_t af = __builtin_bit_cast(
+                h8_t, *(const uint4*)(slab[buf] + ((g * MB + mb) * 4 + b) * 1024 + lane * 16));
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[t], acc[t][mb], 0, 0, 0);
+          }
+        }
+    };
+    // a wave with two tiles and one with a single tile run the same stages
+    auto loop = [&](auto both) __attribute__((always_inline)) {
+      constexpr int NT = decltype(both)::value ? 2 : 1;
+      Lines wa[2], wb[2];
+      load_x(even, 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) load_w(wa[t], t, 0);
+      load_x(odd, 1);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) load_w(wb[t], t, 1);
+      store_x(even, 0);
+      for (int s = 0; s < stages; s += 2) {
+        load_x(even, s + 2);
+        __syncthreads();
+        run(wa, 0, both);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) load_w(wa[t], t, s + 2);
+        store_x(odd, 1);
+        load_x(odd, s + 3);
+        __syncthreads();
+        run(wb, 1, both);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) load_w(wb[t], t, s + 3);
+        store_x(even, 0);
+      }
+      __syncthreads();  // (the next pass fills the slabs again)
+    };
+    if (two) loop(std::true_type());
+    else loop(std::false_type());
+
+    const int col = lane & 15, rq4 = 4 * (lane >> 4);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int at = wave + kWaves * t;
+      if (at >= n) break;
+      const int row = (t0 + p0 + at) * kTileRows + col;
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const int4 e4 = *(const int4*)(a.rexp + 16 * mb + rq4);
+        const int e[4] = {e4.x, e4.y, e4.z, e4.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 16 * mb + rq4 + i;
+          const float v = ldexp_f(acc[t][mb][i], -e[i]);
+          if (a.epi.act == kEpiSwiGLU) {  // n % 16 == 0: every row exists
+            const float p = add_bias(a.epi, v, row);
+            const float up = dpp<kDppRor8>(p);
+            if ((lane & 8) == 0 && r < a.m)
+              a.y[(size_t)r * a.ny + glu_col(row)] = silu_f(p) * up;
+          } else if (r < a.m && row < a.n) {
+            a.y[(size_t)r * a.n + row] = add_bias(a.epi, v, row);
+          }
+        }
+      }
+    }
+  }
+}
+
 // ---- m <= 16: fp32 x read by the kernel itself --------------------------------
 // One row block, so every workgroup's x is 16 rows x its K range: reading
 // it as fp32 costs twice the L2 -> CU bytes of the fp16 copy, but saves the
@@ -502,8 +655,20 @@ int g_tiles_override = 0;   // mlq_set_skinny_plan; 0 = planner
 int g_splits_override = 0;
 
 struct SkinnyPlan {
-  int tiles, splits;
+  int tiles, splits;  // tiles 0: skinny_wide_kernel
 };
+
+// x through LDS from five tiles per CU on, where most of its eight waves have a
+// tile (4 layers of hidden 3584, FFN 18944, us without and with it: 20 rows of
+// q4_0 322, 294, 64 rows 432, 400, 64 rows of q8_0 535, 463; hidden 4096, FFN
+// 14336, 40 rows of q4_1 370, 349). With 704 tiles it loses (hidden 2048, FFN
+// 5632, 64 rows of q4_0 188, 215).
+bool uses_wide(int m, int nt, int g) {
+  if (g_tiles_override != 0 || g_splits_override != 0) return false;
+  // 32-bit buffer offsets into the copy of x, two stages past its end too
+  if ((uint64_t)(g + 8) * ((m + 15) / 16) * 4096 >= (1ull << 31)) return false;
+  return nt >= 5 * device_cus();
+}
 
 // Weight tiles per workgroup (T) and K ranges per tile group (S). A
 // workgroup reads its K range of x once for all of its T tiles, so per CU
@@ -528,6 +693,7 @@ SkinnyPlan skinny_plan(int type, int m, int n, int k) {
   // one-tile one (q4_0 M = 16: 4096 x 4096 7.7 vs 8.8 us, one round
   // either way; 4608 x 3584, 288 tiles: 13.8 us in two rounds vs 9.5 in one)
   const bool x32 = uses_x32(m, k);
+  if (!x32 && uses_wide(m, geo.nt, geo.g)) return SkinnyPlan{0, 1};
   if (x32 && g_tiles_override == 0 && g_splits_override == 0) {
     int t = 1;
     if (type == MLQ_Q4_0) {
@@ -608,6 +774,16 @@ hipError_t launch_typed(const SkinnyArgs& a, int tiles, hipStream_t stream) {
     }
     const unsigned grid = (unsigned)(a.nt * a.splits);
     skinny_x32_kernel<QT, 1><<<grid, kThreads, 0, stream>>>(a);
+    return hipGetLastError();
+  }
+  if (tiles == 0) {
+    const unsigned grid = (unsigned)std::min(a.nt, device_cus());
+    switch ((a.m + 15) / 16) {
+      case 1: skinny_wide_kernel<QT, 1><<<grid, kThreads, 0, stream>>>(a); break;
+      case 2: skinny_wide_kernel<QT, 2><<<grid, kThreads, 0, stream>>>(a); break;
+      case 3: skinny_wide_kernel<QT, 3><<<grid, kThreads, 0, stream>>>(a); break;
+      default: skinny_wide_kernel<QT, 4><<<grid, kThreads, 0, stream>>>(a); break;
+    }
     return hipGetLastError();
   }
   switch (tiles) {

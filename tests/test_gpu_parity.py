@@ -802,3 +802,34 @@ def test_aos_many_tiles(pkg, cuda, qtype, m, n, k):
         buf[lead:lead + raw.numel()] = raw
         y = pkg.linear_aos(qtype, buf[lead:lead + raw.numel()], n, k, x).view(m, n).double()
         assert bool(((y - ref).abs() <= bound).all()), lead
+
+
+# 17..64 rows (and 9..16 too long for the kernels that read fp32 x) with five or more weight tiles per CU:
+# x through LDS, waves with one and two tiles, more than 16 tiles in a workgroup (a second pass), odd
+# group counts, ragged K and N, every count of 16-row blocks.
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("m,n,k", [(17, 20480, 100), (64, 20501, 260), (33, 32016, 516), (48, 65552, 132),
+                                   (20, 40960, 128), (12, 20480, 6148)])
+def test_skinny_many_tiles(pkg, cuda, qtype, m, n, k):
+    import torch
+    from synthetic import synth
+    _print_case(test="skinny_many_tiles", qtype=qtype, m=m, n=n, k=k)
+    g = torch.Generator(device=cuda).manual_seed(m + n + k)
+    tw = pkg.repack_device(qtype, synth.device_blocks(torch, g, qtype, n, k, 0.02, cuda).view(-1).view(torch.uint8), n, k)
+    x = torch.randn((m, k), generator=g, device=cuda)
+    x[0] *= 1e12
+    x[m - 1] *= 1e-12
+    bias = torch.randn(n, generator=g, device=cuda)
+    w64, x64 = pkg.dequantize(tw).double(), x.double()
+    ref = x64 @ w64.t().contiguous() + bias.double()
+    # x and W rounded to fp16 once
+    e = 2.0 ** -10 * (x64.abs() @ w64.abs().t().contiguous() + bias.abs().double())
+    y = pkg.linear(tw, x, bias=bias).double()
+    assert bool(((y - ref).abs() <= e).all())
+    if n % 16 == 0:
+        t, e = ref.view(m, n // 16, 2, 8), e.view(m, n // 16, 2, 8)
+        gate, up = t[:, :, 0], t[:, :, 1]
+        y = pkg.linear(tw, x, bias=bias, act=pkg.EPI_SWIGLU).double().view(m, n // 16, 8)
+        slack = 1.1 * e[:, :, 0] * (up.abs() + e[:, :, 1]) + gate.abs() * e[:, :, 1]
+        slack = slack + 16 * 2.0 ** -23 * (gate * up).abs() + 1e-30
+        assert bool(((y - torch.nn.functional.silu(gate) * up).abs() <= slack).all())
