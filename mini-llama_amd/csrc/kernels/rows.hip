@@ -27,6 +27,8 @@
 //    element by element in fp32 they were bound by ~5 VALU per weight: one
 //    row of 18944 x 3584 q4_0 25.4 -> 13.1 us, q8_0 24.2 -> 15.8, q4_1 24.0 ->
 //    13.9; four rows 88.5 -> 14.1.
+//  - Up to 8 rows longer than the LDS on at most a tile per CU (down
+//    projections): x in pieces, a wave's sums staying in registers.
 //  - Each (row, 128-k group) is scaled by its own power of two (the group's
 //    largest |x| into [2^14, 2^15)) before it becomes fp16, and the group's
 //    sums are scaled back in fp32: any finite x, and no dependence on how
@@ -66,6 +68,7 @@ struct RowsArgs {
   int m, n, k, g, ny;
   int nb, row_bytes;  // kAos*
   int tiles, extra;  // tiles per workgroup; the first `extra` have one more
+  int phase;         // groups staged at a time (all of them, or one tile per workgroup)
   Epilogue epi;
 };
 
@@ -140,7 +143,8 @@ __device__ __forceinline__ float group_max_nonneg(float v) {
   return __builtin_bit_cast(float, b);
 }
 
-template <int QT, int RP, bool HL, int SRC>
+// PH: x in pieces of a.phase groups, one tile per workgroup.
+template <int QT, int RP, bool HL, int SRC, bool PH>
 __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
   using L = Lds<QT, RP, HL>;
   constexpr int MR = L::kRows;
@@ -152,8 +156,8 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
   constexpr bool SUMS = HL && QT == MLQ_Q4_1;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   uint8_t* frag = smem;
-  float* scale = (float*)(smem + (size_t)a.g * L::kGroup);
-  float* sums = (float*)((uint8_t*)scale + (size_t)a.g * L::kScale);
+  float* scale = (float*)(smem + (size_t)a.phase * L::kGroup);
+  float* sums = (float*)((uint8_t*)scale + (size_t)a.phase * L::kScale);
   float* part = (float*)smem;
 
   const int lane = threadIdx.x & 63;
@@ -162,22 +166,22 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
   // this workgroup's tiles and this wave's run of their units
   const int T = a.tiles + ((int)blockIdx.x < a.extra ? 1 : 0);
   const int t0 = (int)blockIdx.x * a.tiles + min((int)blockIdx.x, a.extra);
-  const int U = T * G;
-  const int u0 = wave * U / W, u1 = (wave + 1) * U / W;
-  const int n = u1 - u0;
+  const int U = PH ? a.phase : T * G;
+  int u0 = wave * U / W, u1 = (wave + 1) * U / W, n = u1 - u0;
+  int gb = 0, ge = G;  // the groups in LDS
 
   using U1 = Unit<SRC>;
   constexpr uint32_t QB = QT == MLQ_Q8_0 ? 2048u : 1024u;
   constexpr int BS = aos_block_bytes<QT>();
-  const size_t unit0 = (size_t)t0 * G + u0;
+  size_t unit0 = (size_t)t0 * G + u0;
   const size_t rows0 = (size_t)t0 * kTileRows;
   const uint8_t* aos = a.qs + rows0 * a.row_bytes;  // (kAos*)
   const int lead = SRC == kAos2 ? (int)((uintptr_t)aos & 3) : 0;
-  const rsrc_t rq =
+  rsrc_t rq =
       SRC == kTiled ? make_rsrc(a.qs + unit0 * QB, (uint32_t)n * QB)
                     : make_rsrc(aos - lead, (uint32_t)((lead + (size_t)min((size_t)T * kTileRows, a.n - rows0) * a.row_bytes + 3) & ~(size_t)3));
-  const rsrc_t rd = SRC == kTiled ? make_rsrc(a.d + unit0 * 128, (uint32_t)n * 128u) : rq;
-  const rsrc_t rm = SRC == kTiled && QT == MLQ_Q4_1
+  rsrc_t rd = SRC == kTiled ? make_rsrc(a.d + unit0 * 128, (uint32_t)n * 128u) : rq;
+  rsrc_t rm = SRC == kTiled && QT == MLQ_Q4_1
                         ? make_rsrc(a.mn + unit0 * 128, (uint32_t)n * 128u) : rd;
   const uint32_t qoff = (uint32_t)lane * 16u, soff = (uint32_t)(lane & 15) * 8u;
   // (kAos*) byte offset of the lane's row and the quarter's eight code bytes
@@ -290,12 +294,13 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
       // keep e = 127 (they land below 2^15, coarser but finite)
       const int e = min(pow2_scale_exp(group_max_nonneg<LPR>(mx)), 127);
       const float sc = ldexp_f(1.0f, e);
-      if (g >= G) continue;
-      if (q == 0) scale[g * RP + rho] = ldexp_f(1.0f, -e);
+      if (g >= ge) continue;
+      const int at = PH ? g - gb : g;
+      if (q == 0) scale[at * RP + rho] = ldexp_f(1.0f, -e);
 #pragma unroll
       for (int j = 0; j < NL; ++j) {
         const int f = j * LPR + q;  // float4 of the group: block f / 8, quarter (f / 2) % 4
-        uint8_t* p = frag + (size_t)g * L::kGroup +
+        uint8_t* p = frag + (size_t)at * L::kGroup +
                      (((f >> 3) * 4 + ((f >> 1) & 3)) * MR) * 16 + (f & 1) * 8;
         float4 v = b.v[i][j];
         v.x *= sc;
@@ -311,7 +316,7 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
           if constexpr (SUMS) {
             // (the lanes of a block share their group, so all of them are here)
             const float s = row_sum<8>((v.x + v.y) + (v.z + v.w));
-            if ((f & 7) == 0) sums[(g * kGroupBlocks + (f >> 3)) * RP + rho] = s;
+            if ((f & 7) == 0) sums[(at * kGroupBlocks + (f >> 3)) * RP + rho] = s;
           }
         } else {
           *(uint2*)(p + rho * 16) = make_uint2(pack_h2(v.x, v.y), pack_h2(v.z, v.w));
@@ -320,19 +325,23 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
     }
   };
   // x is requested ahead of the weights (loads return in order and x mostly
-  // hits L2); rows of more than 4096 stage the rest behind them
+  // hits L2); groups past the first 32 are staged behind them
   Batch b0;
-  const int gs = wave * BG;
-  load_x(b0, gs);
   U1 ring[D];
+  auto fill = [&]() __attribute__((always_inline)) {
+    const int gs = gb + wave * BG;
+    load_x(b0, gs);
 #pragma unroll
-  for (int i = 0; i < D; ++i) load(ring[i], i);
-  stage(b0, gs);
-  for (int g = gs + W * BG; g < G; g += W * BG) {
-    load_x(b0, g);
-    stage(b0, g);
-  }
-  __syncthreads();
+    for (int i = 0; i < D; ++i) load(ring[i], i);
+    stage(b0, gs);
+    for (int g = gs + W * BG; g < ge; g += W * BG) {
+      load_x(b0, g);
+      stage(b0, g);
+    }
+    __syncthreads();
+  };
+  if constexpr (PH) ge = min(G, a.phase);
+  fill();
 
   // ---- the wave's units
   float acc[AC], head[AC];  // running; the run's first tile if not whole
@@ -403,23 +412,47 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[i] += p[i] * sc[i];
     }
-    if (++g == G) {
-      flush();
-      g = 0;
-      ++tile;
+    ++g;
+    if constexpr (!PH) {
+      if (g == G) {
+        flush();
+        g = 0;
+        ++tile;
+      }
     }
   };
-  int j = 0;
-  for (; j + D <= n; j += D) {
+  auto stream = [&]() __attribute__((always_inline)) {
+    int j = 0;
+    for (; j + D <= n; j += D) {
 #pragma unroll
-    for (int i = 0; i < D; ++i) {
-      run(ring[i]);
-      load(ring[i], j + D + i);
+      for (int i = 0; i < D; ++i) {
+        run(ring[i]);
+        load(ring[i], j + D + i);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+      if (j + i < n) run(ring[i]);
+  };
+  stream();
+  if constexpr (PH) {
+    // the tile's next groups; each wave keeps its sums
+    for (gb = a.phase; gb < G; gb += a.phase) {
+      ge = min(G, gb + a.phase);
+      const int c = ge - gb;
+      u0 = wave * c / W;
+      u1 = (wave + 1) * c / W;
+      n = u1 - u0;
+      g = u0;
+      unit0 = (size_t)t0 * G + gb + u0;
+      rq = make_rsrc(a.qs + unit0 * QB, (uint32_t)n * QB);
+      rd = make_rsrc(a.d + unit0 * 128, (uint32_t)n * 128u);
+      rm = QT == MLQ_Q4_1 ? make_rsrc(a.mn + unit0 * 128, (uint32_t)n * 128u) : rd;
+      __syncthreads();  // every wave is done with the fragments
+      fill();
+      stream();
     }
   }
-#pragma unroll
-  for (int i = 0; i < D; ++i)
-    if (j + i < n) run(ring[i]);
   // A run's partial tiles: the first one (head, or acc if the run ends inside
   // it) in slot 0, the last one in slot 1.
   __syncthreads();  // every wave is done with the fragments
@@ -434,6 +467,18 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
   __syncthreads();
 
   // ---- tiles shared by several waves, added in wave order
+  if constexpr (PH) {
+    if (wave != 0) return;
+    float v[AC];
+#pragma unroll
+    for (int i = 0; i < AC; ++i) v[i] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+#pragma unroll
+      for (int i = 0; i < AC; ++i) v[i] += part[(w * 2 * 64 + lane) * AC + i];
+    store_tile(v, 0);
+    return;
+  }
   for (int t = wave; t < T; t += W) {
     const int wlo = t * W / T, whi = ((t + 1) * W - 1) / T;  // waves whose runs may meet it
     float v[AC];
@@ -453,15 +498,26 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
   }
 }
 
+size_t lds_limit();
+
 template <int QT, int RP, bool HL, int SRC = kTiled>
 hipError_t launch_rp(RowsArgs a, int nt, hipStream_t stream) {
-  const size_t lds = Lds<QT, RP, HL>::bytes(a.g);
-  const auto kernel = rows_kernel<QT, RP, HL, SRC>;
-  const hipError_t e = allow_dynamic_lds((const void*)kernel, lds);
-  if (e != hipSuccess) return e;
+  using L = Lds<QT, RP, HL>;
   const int grid = std::min(nt, device_cus());
   a.tiles = nt / grid;
   a.extra = nt % grid;
+  a.phase = a.g;
+  void (*kernel)(RowsArgs) = rows_kernel<QT, RP, HL, SRC, false>;
+  if constexpr (SRC == kTiled && HL) {
+    if (L::bytes(a.g) > lds_limit()) {  // (one tile per workgroup, rows_supported)
+      const int most = (int)(lds_limit() / (L::bytes(64) / 64)), pieces = (a.g + most - 1) / most;
+      a.phase = (a.g + pieces - 1) / pieces;
+      kernel = rows_kernel<QT, RP, HL, SRC, true>;
+    }
+  }
+  const size_t lds = L::bytes(a.phase);
+  const hipError_t e = allow_dynamic_lds((const void*)kernel, lds);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), lds, stream, a);
   return hipGetLastError();
 }
@@ -496,9 +552,6 @@ hipError_t launch_aos_qt(const RowsArgs& a, int nt, hipStream_t stream) {
   return four ? launch_aos_src<QT, kAos4>(a, nt, stream) : launch_aos_src<QT, kAos2>(a, nt, stream);
 }
 
-}  // namespace
-
-namespace {
 size_t lds_limit() {
   static const size_t limit = [] {
     int dev = 0, bytes = 0;
@@ -537,7 +590,11 @@ bool rows_supported(int type, int m, int n, int k) {
   const size_t lds = type == MLQ_Q8_0   ? lds_qt<MLQ_Q8_0>(m, g)
                      : type == MLQ_Q4_0 ? lds_qt<MLQ_Q4_0>(m, g)
                                         : lds_qt<MLQ_Q4_1>(m, g);
-  return lds <= lds_limit();
+  // Up to 8 rows on at most a tile per CU take a longer x in pieces (4 rows
+  // of 4096 x 14336 q4_1, 4 layers with it 214 us, 202 in pieces; before that
+  // these ran on fp16 activations; 9..16 rows lose: 16 of 4096 x 14336 q8_0
+  // 288 with the fp16 copy, 302 in pieces).
+  return lds <= lds_limit() || (m <= 8 && geometry(n, k).nt <= device_cus());
 }
 
 hipError_t launch_rows(const mlq_weight& w, const float* x, float* y, int m, hipStream_t stream,

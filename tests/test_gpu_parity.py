@@ -755,7 +755,9 @@ def test_cpp_interface_tests(pkg):
 @pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("m,n,k", [(5, 5137, 100), (8, 5136, 132), (9, 5152, 36), (16, 5121, 4100), (12, 8208, 4864),
                                    (8, 9001, 4736), (16, 40000, 256), (2, 8209, 8196), (3, 16401, 4096),
-                                   (4, 16400, 4228), (2, 3584, 17408), (3, 640, 9216), (6, 100, 4864)])
+                                   (4, 16400, 4228), (2, 3584, 17408), (3, 640, 9216), (6, 100, 4864),
+                                   # x in two, three and five pieces
+                                   (4, 4096, 14336), (8, 100, 9860), (5, 4090, 18948), (2, 48, 40004)])
 def test_resident_rows(pkg, cuda, qtype, m, n, k):
     import torch
     from synthetic import synth
