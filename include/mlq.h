@@ -138,7 +138,10 @@ int mlq_quantize_act_q8_0(const float* x, int rows, int row_size, void* out,
 /* ---------------------------------------------------------------------- */
 
 /* Tiled weight (from the upload path). Picks the kernel family by m:
- *  m = 1..8 (decode): HBM-streaming GEMV, fp32-class accuracy. One row:
+ *  m = 1..8 (decode): HBM-streaming GEMV, fp32-class accuracy; with many
+ *    weight tiles, or an x too long for its staging, 2..8 (and with many
+ *    tiles 9..16) rows stream past an x kept in LDS, same accuracy for their
+ *    row count. One row:
  *    activations as integers (22 bits below the largest |x| of each K
  *    slice, three fp16 digits), codes fed with their fp16 bias and the
  *    bias removed on the matrix core, every block sum exact; several rows
@@ -154,8 +157,8 @@ int mlq_linear(const mlq_weight* w, const float* x, float* y, int m,
 
 /* Device workspace bytes mlq_linear_ws needs for m activation rows with
  * weight w (*bytes = 0 when the kernels for that shape need none: the decode
- * GEMV, and 9..16 rows with k <= 6144, k % 4 == 0, whose skinny kernel reads
- * fp32 x itself). The skinny (17..64 rows, or longer rows) and prefill
+ * GEMV and the resident-x kernel (most calls of 2..8 rows), and 9..16 rows
+ * with k <= 6144, k % 4 == 0, whose skinny kernel reads fp32 x itself). The skinny (17..64 rows, or longer rows) and prefill
  * GEMMs use it for a one-pass fp16 copy of x, which halves the activation
  * bytes their stages move; both also for fp32 partial outputs when they
  * split K across workgroups (shapes with few output tiles). The size
@@ -265,10 +268,11 @@ int mlq_gguf_upload(const mlq_gguf* g, int64_t index, void* aos_dev, size_t aos_
  * (src/cuda_quant.cu:300-361). Up to 8 rows of x whose k fits the kernel's
  * LDS staging (mlq_linear_aos_workspace reports 0 bytes) run a GEMV that
  * reads the blocks as they are, every weight byte once; `workspace` may
- * then be NULL. Otherwise the blocks are repacked into `workspace` (device,
+ * then be NULL. aos_dev is 2-byte aligned, as the blocks are. Otherwise the blocks are repacked into `workspace` (device,
  * >= mlq_weight_layout(...).bytes) and run through mlq_linear. Results
- * meet the Linear's tolerance either way (the direct GEMV sums in fp32
- * like the reference's per-element loop, in another order). */
+ * meet the Linear's tolerance either way (the direct GEMV is fp32-class like
+ * the reference's per-element loop: activations to 2^-22, exact codes, fp32
+ * scales and sums). */
 int mlq_linear_aos(int type, const void* aos_dev, size_t block_count, int n,
                    int k, const float* x, float* y, int m, void* workspace,
                    size_t workspace_bytes, mlq_stream_t stream);
@@ -337,7 +341,8 @@ int mlq_add_bias(float* y, const float* bias, int m, int n,
 /* F32 Linear weights use mlq_weight with type MLQ_F32: base holds W [n][k]
  * fp32 row-major (mlq_weight_layout(MLQ_F32, n, k) gives bytes = 4nk, every
  * offset 0). mlq_linear, mlq_linear_ws and mlq_linear_epi then run an fp32
- * HBM-streaming GEMV (any m, no workspace, same epilogues), replacing the
+ * HBM-streaming GEMV (up to 8 rows) or fp32 MFMA (more; no workspace, same
+ * epilogues), replacing the
  * cuBLAS Sgemm of cudaLinearDeviceInput (src/cuda_matmul.cc:205-241) and the
  * F32 arm of forwardLinearDevice (src/forward.cc:206-209). The GEMM path
  * override (MLQ_PATH_MFMA) is MLQ_ERR_UNSUPPORTED for them. */
