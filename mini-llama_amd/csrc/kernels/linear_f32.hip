@@ -24,8 +24,13 @@
 //    bound by the reads of W (and of x from L2).
 // An MFMA adds to its accumulator in k order, so one chain over all of K
 // would round K times (about 1.5e-6 relative at K = 4096, where the GEMV's 64
-// interleaved lanes give 1.6e-7). Both kernels therefore close a chain every
-// 32 k and add it to a second level, the tiled one to a third every 256 k.
+// interleaved lanes and their tree give 1.6e-7). Both kernels therefore run
+// short chains from zero and add them as trees: of 4 k, as the GEMV's lanes at
+// K = 256, and in the tiled kernel from K = 1024 on of 8 k, which is closer
+// than the GEMV there and takes half the additions. Modelled error, GEMV
+// against tiled and skinny: K = 256 7.7e-8, 7.9e-8, 7.9e-8; 512 8.5e-8,
+// 8.4e-8, 8.2e-8; 1024 9.9e-8, 9.1e-8, 8.7e-8; 4096 1.6e-7, 1.0e-7, 1.1e-7
+// (chains of 32 k: 1.2e-7 at 256 and 512).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -155,7 +160,8 @@ constexpr int kTile = 64, kStageK = 32, kLdsRow = kStageK + 4;
 template <int KS>
 constexpr int gemm_f32_lds() { return KS * 2 * 2 * kTile * kLdsRow * (int)sizeof(float); }
 
-template <int KS, bool VEC>
+// CH: k of a chain (4 or 8).
+template <int KS, bool VEC, int CH>
 __global__ __launch_bounds__(256 * KS) void gemm_f32_kernel(F32Args a) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -197,17 +203,25 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_kernel(F32Args a) {
   f16v_t sum = {}, mid = {};
   const int frag = (lane & 31) * kLdsRow + 4 * (lane >> 5);
   const int arow = 32 * wm * kLdsRow + frag, brow = (kTile + 32 * wn) * kLdsRow + frag;
-  auto run = [&](int buf) __attribute__((always_inline)) {
-    const float* p = slab + buf * 2 * kTile * kLdsRow;
-    f16v_t in = {};
+  // the sum over 8 k, as one chain or two
+  auto eight = [&](const float* p) __attribute__((always_inline)) {
+    const f4_t av = *(const f4_t*)(p + arow), bv = *(const f4_t*)(p + brow);
+    f16v_t c[8 / CH];
 #pragma unroll
-    for (int j = 0; j < kStageK / 8; ++j) {
-      const f4_t av = *(const f4_t*)(p + arow + 8 * j), bv = *(const f4_t*)(p + brow + 8 * j);
+    for (int q = 0; q < 8 / CH; ++q) {
+      c[q] = (f16v_t){};
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        in = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], in, 0, 0, 0);
+      for (int i = q * CH / 2; i < (q + 1) * CH / 2; ++i)
+        c[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], c[q], 0, 0, 0);
     }
-    mid += in;
+    if constexpr (CH == 4) c[0] += c[1];
+    return c[0];
+  };
+  auto run = [&](int buf) __attribute__((always_inline)) {
+    static_assert(kStageK == 32, "four sums of 8 k");
+    const float* p = slab + buf * 2 * kTile * kLdsRow;
+    const f16v_t lo = eight(p) + eight(p + 8);
+    return lo + (eight(p + 16) + eight(p + 24));
   };
   // stages past the part's end (an odd count, or the last prefetches) load
   // zeros and add nothing
@@ -217,12 +231,13 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_kernel(F32Args a) {
   for (int s = 0; s < per_ks; s += 2) {
     load(even, s + 2);
     __syncthreads();
-    run(0);
+    f16v_t two = run(0);
     store(odd, 1);
     load(odd, s + 3);
     __syncthreads();
-    run(1);
+    two += run(1);
     store(even, 0);
+    mid += two;
     if ((s & 6) == 6) {
       sum += mid;
       mid = (f16v_t){};
@@ -302,18 +317,18 @@ __global__ __launch_bounds__(64 * kSkinnyF32Waves) void skinny_f32_kernel(F32Arg
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) acc[mb] = (f4_t){0.f, 0.f, 0.f, 0.f};
   auto run = [&](const Block& b) __attribute__((always_inline)) {
-    f4_t in[MB];
+    const f4_t z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) in[mb] = (f4_t){0.f, 0.f, 0.f, 0.f};
+    for (int mb = 0; mb < MB; ++mb) {
+      f4_t in[2][4];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-          in[mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x[mb][h][i], b.w[h][i], in[mb], 0, 0, 0);
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[mb] += in[mb];
+        for (int i = 0; i < 4; ++i)
+          in[h][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x[mb][h][i], b.w[h][i], z, 0, 0, 0);
+      acc[mb] += ((in[0][0] + in[0][1]) + (in[0][2] + in[0][3])) +
+                 ((in[1][0] + in[1][1]) + (in[1][2] + in[1][3]));
+    }
   };
   Block b0, b1;
   load(b0, 0);
@@ -332,10 +347,9 @@ __global__ __launch_bounds__(64 * kSkinnyF32Waves) void skinny_f32_kernel(F32Arg
       part[((wave * MB + mb) * 16 + 4 * (lane >> 4) + i) * 16 + (lane & 15)] = acc[mb][i];
   __syncthreads();
   auto total = [&](int r, int c) {
-    float s = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kSkinnyF32Waves; ++w) s += part[(w * 16 * MB + r) * 16 + c];
-    return s;
+    static_assert(kSkinnyF32Waves == 8, "a tree of eight");
+    auto at = [&](int w) { return part[(w * 16 * MB + r) * 16 + c]; };
+    return ((at(0) + at(1)) + (at(2) + at(3))) + ((at(4) + at(5)) + (at(6) + at(7)));
   };
   if (a.epi.act == kEpiSwiGLU) {
     for (int o = tid; o < mr * 8; o += 64 * kSkinnyF32Waves) {
@@ -364,7 +378,7 @@ hipError_t launch_mfma_f32(const F32Args& a, hipStream_t s) {
   if (linear_f32_tiled(a.m, a.n)) {
     const int tiles = ((a.m + kTile - 1) / kTile) * ((a.n + kTile - 1) / kTile);
     constexpr int KS = 2;
-    const auto kernel = gemm_f32_kernel<KS, VEC>;
+    const auto kernel = a.k < 1024 ? gemm_f32_kernel<KS, VEC, 4> : gemm_f32_kernel<KS, VEC, 8>;
     const hipError_t e = allow_dynamic_lds((const void*)kernel, gemm_f32_lds<KS>());
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3((tiles + 7) / 8 * 8), dim3(256 * KS), gemm_f32_lds<KS>(), s, a);
