@@ -26,10 +26,12 @@
 // would round K times (about 1.5e-6 relative at K = 4096, where the GEMV's 64
 // interleaved lanes and their tree give 1.6e-7). Both kernels therefore run
 // short chains from zero and add them as trees: of 4 k, as the GEMV's lanes at
-// K = 256, and in the tiled kernel from K = 1024 on of 8 k, which is closer
-// than the GEMV there and takes half the additions. Modelled error, GEMV
-// against tiled and skinny: K = 256 7.7e-8, 7.9e-8, 7.9e-8; 512 8.5e-8,
-// 8.4e-8, 8.2e-8; 1024 9.9e-8, 9.1e-8, 8.7e-8; 4096 1.6e-7, 1.0e-7, 1.1e-7
+// K = 256; in the tiled kernel of 16 k from K = 1536 and of 32 k from K = 3072,
+// where the GEMV's own chains have grown past them (every chain that is cut
+// costs 16 additions per lane: 200 x 4096 x 4096 takes 91 us in chains of 8).
+// Modelled error, GEMV against tiled and skinny: K = 256 7.7e-8, 7.9e-8,
+// 7.9e-8; 512 8.8e-8, 8.4e-8, 8.4e-8; 1536 1.11e-7, 1.07e-7, 9.7e-8; 3072
+// 1.42e-7, 1.24e-7, 1.03e-7; 4096 1.55e-7, 1.25e-7, 1.07e-7
 // (chains of 32 k: 1.2e-7 at 256 and 512).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -160,7 +162,7 @@ constexpr int kTile = 64, kStageK = 32, kLdsRow = kStageK + 4;
 template <int KS>
 constexpr int gemm_f32_lds() { return KS * 2 * 2 * kTile * kLdsRow * (int)sizeof(float); }
 
-// CH: k of a chain (4 or 8).
+// CH: k of a chain (4, 16 or 32).
 template <int KS, bool VEC, int CH>
 __global__ __launch_bounds__(256 * KS) void gemm_f32_kernel(F32Args a) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -203,25 +205,27 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_kernel(F32Args a) {
   f16v_t sum = {}, mid = {};
   const int frag = (lane & 31) * kLdsRow + 4 * (lane >> 5);
   const int arow = 32 * wm * kLdsRow + frag, brow = (kTile + 32 * wn) * kLdsRow + frag;
-  // the sum over 8 k, as one chain or two
-  auto eight = [&](const float* p) __attribute__((always_inline)) {
-    const f4_t av = *(const f4_t*)(p + arow), bv = *(const f4_t*)(p + brow);
-    f16v_t c[8 / CH];
-#pragma unroll
-    for (int q = 0; q < 8 / CH; ++q) {
-      c[q] = (f16v_t){};
-#pragma unroll
-      for (int i = q * CH / 2; i < (q + 1) * CH / 2; ++i)
-        c[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], c[q], 0, 0, 0);
-    }
-    if constexpr (CH == 4) c[0] += c[1];
-    return c[0];
-  };
   auto run = [&](int buf) __attribute__((always_inline)) {
-    static_assert(kStageK == 32, "four sums of 8 k");
     const float* p = slab + buf * 2 * kTile * kLdsRow;
-    const f16v_t lo = eight(p) + eight(p + 8);
-    return lo + (eight(p + 16) + eight(p + 24));
+    // MFMA u takes two k: the chain it belongs to starts every CH / 2
+    f4_t av, bv;
+    f16v_t c[32 / CH];
+#pragma unroll
+    for (int u = 0; u < kStageK / 2; ++u) {
+      if (u % 4 == 0) {
+        av = *(const f4_t*)(p + arow + 2 * u);
+        bv = *(const f4_t*)(p + brow + 2 * u);
+      }
+      f16v_t& in = c[u / (CH / 2)];
+      if (u % (CH / 2) == 0) in = (f16v_t){};
+      in = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u % 4], bv[u % 4], in, 0, 0, 0);
+    }
+    if constexpr (CH == 4) {
+      c[0] = (c[0] + c[1]) + (c[2] + c[3]);
+      c[1] = (c[4] + c[5]) + (c[6] + c[7]);
+    }
+    if constexpr (CH < 32) c[0] += c[1];
+    return c[0];
   };
   // stages past the part's end (an odd count, or the last prefetches) load
   // zeros and add nothing
@@ -378,7 +382,9 @@ hipError_t launch_mfma_f32(const F32Args& a, hipStream_t s) {
   if (linear_f32_tiled(a.m, a.n)) {
     const int tiles = ((a.m + kTile - 1) / kTile) * ((a.n + kTile - 1) / kTile);
     constexpr int KS = 2;
-    const auto kernel = a.k < 1024 ? gemm_f32_kernel<KS, VEC, 4> : gemm_f32_kernel<KS, VEC, 8>;
+    const auto kernel = a.k < 1536   ? gemm_f32_kernel<KS, VEC, 4>
+                        : a.k < 3072 ? gemm_f32_kernel<KS, VEC, 16>
+                                     : gemm_f32_kernel<KS, VEC, 32>;
     const hipError_t e = allow_dynamic_lds((const void*)kernel, gemm_f32_lds<KS>());
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3((tiles + 7) / 8 * 8), dim3(256 * KS), gemm_f32_lds<KS>(), s, a);
