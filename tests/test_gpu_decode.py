@@ -381,7 +381,7 @@ def test_linear_f32_swiglu(pkg, oracle, cuda):
 # rows that start off 16-byte boundaries (k % 4), K parts of unequal and of no length.
 @pytest.mark.parametrize("m,n,k", [(9, 40, 4), (16, 16, 7), (17, 33, 95), (32, 100, 1000), (33, 64, 33),
                                    (64, 50, 2052), (65, 48, 288), (200, 96, 31), (130, 8200, 66),
-                                   (64, 12289, 64), (769, 1040, 36), (1000, 1000, 4097)])
+                                   (64, 12289, 64), (769, 1040, 36), (769, 1040, 2052), (1000, 1000, 4097)])
 @pytest.mark.parametrize("swiglu", [False, True])
 def test_linear_f32_many_rows(pkg, cuda, m, n, k, swiglu):
     import torch
