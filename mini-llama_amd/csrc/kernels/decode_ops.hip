@@ -1257,14 +1257,14 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
 
 // e^(s - m) for s <= m as 2^h (1 + f ln 2), h + f = (s - m) log2 e with h the
 // rounded product and f what it lost (log2 e in two parts): the hardware
-// exp2's own error and no more.
+// exp2's own error and no more. 0 for s = -inf, NaN where expf(s - m) is.
 __device__ __forceinline__ float exp_diff(float s, float m) {
   constexpr float kLog2e = 1.44269504088896341f, kLn2 = 0.693147180559945309f;
   constexpr float kLog2eLow = (float)(1.44269504088896340735992 - (double)kLog2e);
   const float t = s - m, h = t * kLog2e;
   const float f = __builtin_fmaf(t, kLog2eLow, __builtin_fmaf(t, kLog2e, -h));
   const float e = __builtin_amdgcn_exp2f(h);
-  return h > -200.0f ? __builtin_fmaf(e * kLn2, f, e) : 0.0f;  // (-inf: f is NaN)
+  return h > -200.0f ? __builtin_fmaf(e * kLn2, f, e) : e;  // (h -inf: f is NaN, e is 0)
 }
 
 // ---- long caches: keys streamed through fp32 MFMA ----------------------------------

@@ -22,6 +22,7 @@ oracle's):
 from __future__ import annotations
 
 import ctypes
+import math
 import os
 
 import numpy as np
@@ -266,6 +267,70 @@ def test_attention_long_cache(pkg, cuda, n_heads, n_kv, hd, max_seq, pos):
     # scores of about 1 to 2^-22 each way, weights and their sums in fp32
     bound = 2e-6 * (p[:, :, None] * v64.abs()).sum(dim=0)
     assert bool(((out.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,max_seq,pos", [(28, 4, 128, 13000, 12900), (8, 8, 64, 7000, 6900), (16, 1, 256, 50000, 49900)])
+def test_attention_long_cache_non_finite(pkg, cuda, n_heads, n_kv, hd, max_seq, pos):
+    """A streamed key whose score is NaN, +inf or -inf, and an infinite V, give what softmax gives: NaN, NaN, a weight
+    of 0, an infinite output dim."""
+    import torch
+    g = torch.Generator(device=cuda).manual_seed(pos)
+    keys = torch.randn((1, max_seq, n_kv, hd), generator=g, device=cuda)
+    values = torch.randn((1, max_seq, n_kv, hd), generator=g, device=cuda)
+    q = torch.randn((n_heads, hd), generator=g, device=cuda)
+    q[:, 5] = q[:, 5].abs() + 0.1
+    c = pkg.MlqKvCache(keys.data_ptr(), values.data_ptr(), 1, max_seq, n_kv, hd)
+    lib, nbytes = pkg.lib(), ctypes.c_size_t()
+    _ok(pkg, lib.mlq_attention_workspace(ctypes.byref(c), n_heads, ctypes.byref(nbytes)), "ws")
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device=cuda)
+
+    def run():
+        out = torch.empty((n_heads, hd), device=cuda)
+        _ok(pkg, lib.mlq_attention_decode(ctypes.byref(c), 0, pos, q.data_ptr(), n_heads, out.data_ptr(),
+                                          ws.data_ptr(), ws.numel(), _s(pkg)), "attention")
+        return out
+
+    clean = run()
+    assert bool(torch.isfinite(clean).all())
+    group = n_heads // n_kv
+    for at in (0, 77, pos):  # the first, an inner and the last visible position, in the last kv head only
+        for value in (math.nan, math.inf):
+            kept = float(keys[0, at, n_kv - 1, 5])
+            keys[0, at, n_kv - 1, 5] = value
+            out = run()
+            assert bool(torch.isnan(out[-group:]).all()) and torch.equal(out[:-group], clean[:-group]), (at, value)
+            keys[0, at, n_kv - 1, 5] = kept
+    keys[0, 77, n_kv - 1, 5] = -math.inf
+    out = run()
+    seen = torch.arange(pos + 1, device=cuda) != 77
+    k64 = keys[0, :pos + 1, n_kv - 1][seen].double()
+    v64 = values[0, :pos + 1, n_kv - 1][seen].double()
+    p = torch.softmax(q[-group:].double() @ k64.t().contiguous() / hd ** 0.5, dim=1)
+    assert bool(((out[-group:].double() - p @ v64).abs() <= 2e-6 * (p @ v64.abs())).all())
+    keys[0, 77, n_kv - 1, 5] = 0.0
+    values[0, 77, n_kv - 1, 9] = math.inf
+    out = run()
+    assert bool((out[-group:, 9] == math.inf).all())
+    out[-group:, 9] = 0.0
+    assert bool(torch.isfinite(out).all())
+
+
+def test_decode_step_in_a_long_cache_keeps_nan(pkg, cuda):
+    """The same with the position on the device: a NaN key in the past reaches the logits."""
+    import mini_llama_amd.decode as dec
+    from synthetic import synth
+    cfg = dict(vocab_size=200, dim=256, hidden_dim=256, n_layers=1, n_heads=8, n_kv_heads=8, head_dim=128,
+               max_seq_len=9000, rope_type=1)
+    model = dec.DecodeModel(synth.synthetic_model(cfg, "q8_0", seed=4))
+    model.keys.normal_()
+    model.values.normal_()
+    model.keys[0, 4000, 3, 7] = math.nan
+    for pos, finite in ((3999, True), (4000, True), (4001, False), (8999, False)):  # (4000 is written by the step)
+        model.keys[0, 4000, 3, 7] = math.nan
+        model.token_dev.fill_(17)
+        model.pos_dev.fill_(pos)
+        model.step_device()
+        assert bool(model.logits.isfinite().all() if finite else model.logits.isnan().all()), pos
 
 
 @pytest.mark.parametrize("hd,n_heads,n_kv", [(64, 16, 16), (128, 56, 8), (256, 8, 8)])
