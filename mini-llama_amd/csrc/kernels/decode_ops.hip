@@ -2052,6 +2052,36 @@ int attn_hsplit_override() {
   return v;
 }
 
+// Where one row's keys stream through attn_stream_kernel instead of a
+// workgroup per 32 positions. It takes ~7 us longer to start (16 query rows
+// whatever the group, deep loads, a merge in LDS) and reads K and V faster;
+// the register kernel's time grows with the query heads it holds (1, 2, 4,
+// 8, 16) and its combine with the positions. us, register kernel -> this one:
+//  - Groups of 5 and more: past 192 positions x kv heads per CU (28 heads on 4
+//    of 128 at position 30000 65.9 -> 32.3; 64 on 8 at the line 24.2 -> 20.5, of
+//    64 18.2 -> 13.8, of 256 51.1 -> 37.7).
+//  - Groups up to 4 (32 heads on 32 of 128, position 1600: 14.1 -> 19.1; on 8,
+//    6200: 22.2 -> 19.1, but 3 more where RoPE is fused): past that line and,
+//    alone, from 16384 positions at head_dim 64 (8 kv heads 21.3 -> 20.1;
+//    12288 17.0 -> 17.6), 12288 at 128 (36.1 -> 30.2; 8192 23.0 -> 23.3), 4096
+//    at 256 (32 kv heads 70.4 -> 61.8; 2048 36.1 -> 37.6). With the fused RoPE and cache write, a layer of the
+//    step: 24576 at 64 (4 kv heads 35.7 -> 34.6; 16384 31.3 -> 32.3) and 128
+//    (52.6 -> 48.6; 43.1 -> 43.8), 8192 at 256 (8 kv heads 58.7 -> 58.1; 6144
+//    47.8 -> 52.9).
+//  - A device position says only the capacity: past 256 per CU and where a
+//    short position costs nothing either: groups of 5 and more at 64 and 128
+//    (28 heads on 4 in a 32768 cache, a layer: position 20 32.9 -> 32.8, 32767
+//    85.5 -> 62.4; 4 heads on each of 8: 8192 51.6 -> 53.2; 32 on 32, 1100 38.6
+//    -> 46.3; head_dim 256: 5 to 9 us more up to position 1100).
+bool streams_keys(int hd, int group, int n_kv, int max_len, bool fused, bool device_pos) {
+  const int64_t positions = max_len, work = positions * n_kv, cus = device_cus();
+  if (device_pos) return work > 256 * cus && group > 4 && hd <= 128;
+  if (work <= 192 * cus) return false;
+  if (group > 4) return true;
+  return positions >= (fused ? hd == 256 ? 8192 : 24576
+                             : hd == 256 ? 4096 : hd == 128 ? 12288 : 16384);
+}
+
 hipError_t launch_attention(const AttnLaunch& r, hipStream_t stream) {
   AttnArgs a;
   a.q = r.q;
@@ -2105,19 +2135,12 @@ hipError_t launch_attention(const AttnLaunch& r, hipStream_t stream) {
       a.hsplit = (a.group + a.hper - 1) / a.hper;  // no empty split
     }
   }
-  // Long: the keys stream through attn_stream_kernel, two workgroups per CU.
-  // Position 30000 of a 32768 cache, 28 heads on 4 kv heads of 128 (123 MB):
-  // 65.9 -> 32.3 us with its combine (a chunk per workgroup left 938
-  // partials per head, and their combine took longer than the chunks); one
-  // workgroup per CU is the same, three 39.9. The line is 192 positions x kv
-  // heads per CU: below it the register kernel's finer chunks win (32 heads
-  // on 8 kv heads of 128, position 4200: 17.9 us against 18.6; 8000: 25.1
-  // against 20.6). A device position says only the capacity, so there
-  // more than 256: a 7B layer in a 32768 cache takes 0.15 us more at position
-  // 1100 and 33 us less at 30000.
+  // Long: the keys stream through attn_stream_kernel, two workgroups per CU
+  // (one is the same at position 30000 of a 32768 cache, 28 heads on 4 kv
+  // heads of 128; three take 39.9 us against 32.3).
   const bool stream_keys = reg && a.rows == 1 && a.hsplit == 1 &&
-                           (int64_t)r.max_len * a.n_kv >
-                               (r.pos_dev != nullptr ? 256 : 192) * (int64_t)device_cus() &&
+                           streams_keys(r.hd, a.group, r.n_kv, r.max_len, r.rope_cs != nullptr,
+                                        r.pos_dev != nullptr) &&
                            (uint64_t)r.max_seq * r.n_kv * r.hd * 4 < (1ull << 31);
   if (stream_keys) {
     a.chunk_len = 16 * prefill_waves(r.hd);

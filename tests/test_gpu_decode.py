@@ -238,12 +238,15 @@ def test_attention_matches_oracle(pkg, oracle, cuda, n_heads, n_kv, hd, max_seq,
                                atol=1e-5)
 
 
-# Long caches stream their keys (more than 192 positions x kv heads per CU, 256 where the
-# position is on the device): spans of 64 positions (32 at head_dim 256) shared out over the workgroups, so positions
+# Long caches stream their keys (more than 192 positions x kv heads per CU, and with up to 4 heads per kv head
+# 16384 / 12288 / 4096 positions of 64 / 128 / 256): spans of 64 positions (32 at head_dim 256) shared out over the workgroups, so positions
 # at the edges of 16-key steps, of spans and of a workgroup's second span; groups of 1 to 16 heads.
 @pytest.mark.parametrize("n_heads,n_kv,hd,max_seq,pos", [
     (28, 4, 128, 13000, 12287), (28, 4, 128, 13000, 12288), (8, 8, 64, 7000, 6207), (32, 8, 64, 9000, 8207),
-    (64, 4, 128, 13000, 12415), (16, 1, 256, 50000, 49200), (40, 8, 256, 6300, 6159), (12, 2, 128, 25000, 24591)])
+    (64, 4, 128, 13000, 12415), (16, 1, 256, 50000, 49200), (40, 8, 256, 6300, 6159), (12, 2, 128, 25000, 24591),
+    # groups of 1, 3 and 4 on both sides of their lines
+    (8, 8, 64, 16400, 16382), (8, 8, 64, 16400, 16383), (24, 8, 128, 13000, 12286), (24, 8, 128, 13000, 12287),
+    (64, 16, 256, 4200, 4095), (1, 1, 128, 49300, 49200)])
 def test_attention_long_cache(pkg, cuda, n_heads, n_kv, hd, max_seq, pos):
     import torch
     g = torch.Generator(device=cuda).manual_seed(pos)
@@ -269,7 +272,7 @@ def test_attention_long_cache(pkg, cuda, n_heads, n_kv, hd, max_seq, pos):
     assert bool(((out.double() - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("n_heads,n_kv,hd,max_seq,pos", [(28, 4, 128, 13000, 12900), (8, 8, 64, 7000, 6900), (16, 1, 256, 50000, 49900)])
+@pytest.mark.parametrize("n_heads,n_kv,hd,max_seq,pos", [(28, 4, 128, 13000, 12900), (8, 8, 64, 17000, 16900), (16, 1, 256, 50000, 49900)])
 def test_attention_long_cache_non_finite(pkg, cuda, n_heads, n_kv, hd, max_seq, pos):
     """A streamed key whose score is NaN, +inf or -inf, and an infinite V, give what softmax gives: NaN, NaN, a weight
     of 0, an infinite output dim."""
@@ -319,7 +322,7 @@ def test_decode_step_in_a_long_cache_keeps_nan(pkg, cuda):
     """The same with the position on the device: a NaN key in the past reaches the logits."""
     import mini_llama_amd.decode as dec
     from synthetic import synth
-    cfg = dict(vocab_size=200, dim=256, hidden_dim=256, n_layers=1, n_heads=8, n_kv_heads=8, head_dim=128,
+    cfg = dict(vocab_size=200, dim=256, hidden_dim=256, n_layers=1, n_heads=40, n_kv_heads=8, head_dim=128,
                max_seq_len=9000, rope_type=1)
     model = dec.DecodeModel(synth.synthetic_model(cfg, "q8_0", seed=4))
     model.keys.normal_()
@@ -333,7 +336,7 @@ def test_decode_step_in_a_long_cache_keeps_nan(pkg, cuda):
         assert bool(model.logits.isfinite().all() if finite else model.logits.isnan().all()), pos
 
 
-@pytest.mark.parametrize("hd,n_heads,n_kv", [(64, 16, 16), (128, 56, 8), (256, 8, 8)])
+@pytest.mark.parametrize("hd,n_heads,n_kv", [(64, 16, 16), (128, 56, 8), (256, 8, 8), (64, 40, 8)])
 def test_decode_step_in_a_long_cache(pkg, cuda, hd, n_heads, n_kv):
     """The device-position step (its grid covers the whole cache, so keys stream and the current row
     is rotated and written by the streaming kernel) against the host-position step."""
