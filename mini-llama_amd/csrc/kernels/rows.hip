@@ -378,6 +378,12 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
 #pragma unroll
     for (int i = 0; i < AC; ++i) acc[i] = 0.0f;
   };
+  // this lane's two rows of p's RP values (one row: its value and nothing past
+  // it, which would be off an 8-byte boundary and, at the end, outside the LDS)
+  auto row_pair = [&](const float* p) __attribute__((always_inline)) {
+    if constexpr (RP == 1) return make_float2(p[0], 0.0f);
+    else return *(const float2*)(p + r0);
+  };
   auto run = [&](const U1& s) __attribute__((always_inline)) {
     const uint8_t* af = af0 + (size_t)g * L::kGroup;
     if constexpr (HL) {
@@ -392,12 +398,12 @@ __global__ __launch_bounds__(64 * W) void rows_kernel(RowsArgs a) {
         t[0] += d * (p[0] + p[1]);
         t[1] += d * (p[2] + p[3]);
         if constexpr (SUMS) {
-          const float2 sx = *(const float2*)(sums + (g * kGroupBlocks + b) * RP + r0);
+          const float2 sx = row_pair(sums + (g * kGroupBlocks + b) * RP);
           t[0] += mb * sx.x;
           t[1] += mb * sx.y;
         }
       }
-      const float2 sc = *(const float2*)(scale + g * RP + r0);
+      const float2 sc = row_pair(scale + g * RP);
       acc[0] += t[0] * sc.x;
       acc[1] += t[1] * sc.y;
     } else {

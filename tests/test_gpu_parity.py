@@ -787,7 +787,9 @@ def test_resident_rows(pkg, cuda, qtype, m, n, k):
 # Raw GGUF blocks with several tiles per workgroup (whole and shared ones), odd block counts (rows off
 # 4-byte boundaries), k % 4 != 0, a base off a 4-byte boundary, blocks of the last group past the row.
 @pytest.mark.parametrize("qtype", TYPES)
-@pytest.mark.parametrize("m,n,k", [(1, 9001, 1056), (3, 8200, 3104), (8, 4500, 994), (1, 20000, 99), (2, 16411, 128)])
+@pytest.mark.parametrize("m,n,k", [(1, 9001, 1056), (3, 8200, 3104), (8, 4500, 994), (1, 20000, 99), (2, 16411, 128),
+                                   # one row of 1, 33 and 65 groups, past the LDS that the partial tiles take
+                                   (1, 64, 96), (1, 64, 4224), (1, 4112, 8320)])
 def test_aos_many_tiles(pkg, cuda, qtype, m, n, k):
     import torch
     from synthetic import synth
