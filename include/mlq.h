@@ -270,9 +270,8 @@ int mlq_gguf_upload(const mlq_gguf* g, int64_t index, void* aos_dev, size_t aos_
  * reads the blocks as they are, every weight byte once; `workspace` may
  * then be NULL. aos_dev is 2-byte aligned, as the blocks are. Otherwise the blocks are repacked into `workspace` (device,
  * >= mlq_weight_layout(...).bytes) and run through mlq_linear. Results
- * meet the Linear's tolerance either way (the direct GEMV is fp32-class like
- * the reference's per-element loop: activations to 2^-22, exact codes, fp32
- * scales and sums). */
+ * meet the Linear's tolerance either way (the direct GEMV dequantizes and sums
+ * in fp32 like the reference's per-element loop, in another order). */
 int mlq_linear_aos(int type, const void* aos_dev, size_t block_count, int n,
                    int k, const float* x, float* y, int m, void* workspace,
                    size_t workspace_bytes, mlq_stream_t stream);

@@ -170,8 +170,8 @@ hipError_t launch_skinny_ws(const mlq_weight& w, const float* x, float* y, int m
 void set_skinny_plan(int tiles, int splits);
 bool skinny_plan_set();
 
-// rows.hip: GEMV straight from GGUF AoS blocks (m <= 8 rows of x, x
-// resident in LDS: aos_gemv_supported says whether the shape fits).
+// aos_gemv.hip: GEMV straight from GGUF AoS blocks (m <= 8 rows of x, x
+// staged in LDS: aos_gemv_supported says whether the shape fits).
 bool aos_gemv_supported(int type, int m, int n, int k);
 hipError_t launch_aos_gemv(int type, const void* aos, int n, int k, const float* x, float* y,
                            int m, hipStream_t stream);

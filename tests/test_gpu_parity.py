@@ -11,6 +11,8 @@ from __future__ import annotations
 
 import os
 
+import math
+
 import numpy as np
 import pytest
 
@@ -788,7 +790,7 @@ def test_resident_rows(pkg, cuda, qtype, m, n, k):
 # 4-byte boundaries), k % 4 != 0, a base off a 4-byte boundary, blocks of the last group past the row.
 @pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("m,n,k", [(1, 9001, 1056), (3, 8200, 3104), (8, 4500, 994), (1, 20000, 99), (2, 16411, 128),
-                                   # one row of 1, 33 and 65 groups, past the LDS that the partial tiles take
+                                   # one row of 1, 33 and 65 groups
                                    (1, 64, 96), (1, 64, 4224), (1, 4112, 8320)])
 def test_aos_many_tiles(pkg, cuda, qtype, m, n, k):
     import torch
@@ -806,6 +808,46 @@ def test_aos_many_tiles(pkg, cuda, qtype, m, n, k):
         buf[lead:lead + raw.numel()] = raw
         y = pkg.linear_aos(qtype, buf[lead:lead + raw.numel()], n, k, x).view(m, n).double()
         assert bool(((y - ref).abs() <= bound).all()), lead
+
+
+# Raw blocks are fp32 per element: what fp32 holds of a weight and an activation reaches the product.
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("m,n", [(1, 48), (2, 48), (3, 48), (8, 48), (1, 8208), (2, 8208)])
+def test_aos_fp32_range(pkg, cuda, qtype, m, n):
+    import torch
+    from synthetic import synth
+    k = 1056
+    g = torch.Generator(device=cuda).manual_seed(m)
+    raw = synth.device_blocks(torch, g, qtype, n, k, 0.02, cuda).view(n, k // 32, -1).view(torch.uint8)
+    zero = {"q8_0": 0x00, "q4_0": 0x88, "q4_1": 0x00}[qtype]  # the code whose weight is 0 (q4_1: with min 0)
+    raw[:, 3, (4 if qtype == "q4_1" else 2):] = zero  # block 3 of every row: weights of 0
+    if qtype == "q4_1":
+        raw[:, 3, 2:4] = 0
+        # blocks 5..: d = 1, q = 7, min = -(7 - 2^-8): weights of 2^-8 whose parts are 1800 times larger
+        raw[:, 5:, :4] = torch.tensor([1.0, -(7.0 - 2.0 ** -8)], dtype=torch.float16, device=cuda).view(torch.uint8)
+        raw[:, 5:, 4:] = 0x77
+    raw = raw.reshape(-1)
+    w64 = pkg.dequantize(pkg.repack_device(qtype, raw, n, k)).double()
+    assert float(w64[:, 96:128].abs().max()) == 0.0
+    x = torch.randn((m, k), generator=g, device=cuda)
+    x[:, 96:128] *= 2.0 ** 60  # meets zero weights only, in the same 128 columns as the activations around it
+    if m > 1:
+        x[0] *= 2.0 ** -60
+        x[m - 1] *= 2.0 ** 60
+    # products rounded never, sums: chains of 16, then 2 + (k / 128) + 2 + 16 additions; a weight's one rounding
+    bound = (16 + 2 + k // 128 + 1 + 2 + 16 + 1) * 2.0 ** -24
+    ref, size = x.double() @ w64.t().contiguous(), x.double().abs() @ w64.abs().t().contiguous()
+    y = pkg.linear_aos(qtype, raw, n, k, x).view(m, n)
+    assert bool(((y.double() - ref).abs() <= bound * size).all())
+    # an infinite activation gives what the fp32 products give, in its row only
+    x[0, 200] = math.inf
+    z = pkg.linear_aos(qtype, raw, n, k, x).view(m, n)
+    w = w64[:, 200]
+    assert bool((z[0][w > 0] == math.inf).all() and (z[0][w < 0] == -math.inf).all() and z[0][w == 0].isnan().all())
+    assert torch.equal(z[1:], y[1:])
+    x[0, 200] = math.nan
+    z = pkg.linear_aos(qtype, raw, n, k, x).view(m, n)
+    assert bool(z[0].isnan().all()) and torch.equal(z[1:], y[1:])
 
 
 # 17..64 rows (and 9..16 too long for the kernels that read fp32 x) with five or more weight tiles per CU:
