@@ -2,37 +2,25 @@
 // the reference uploads them): y[r][n] = sum_k W[n][k] x[r][k] for r < m <= 8,
 // every weight byte read from HBM once, no repack. This is the raw-pointer
 // meaning of the reference's cudaQ*LinearDeviceWeight / DeviceInput weight
-// (src/cuda_quant.cu:300-361), behind mlq_linear_aos.
-//
-// The arithmetic is the reference's per-element dequantization in fp32
-// (src/quant.cc:477-503): every weight becomes the fp32 value d * q, d * (q - 8)
-// (both exact) or d * q + m (rounded once) and meets the fp32 activation in an
-// fp32 multiply-add. fp16 hi + lo pairs of x at the fp16 matrix rate are faster
-// (one row of 18944 x 3584 q4_0 13.1 us) but lose what lies 2^-39 below the
-// largest x of its 128 columns and infinite activations, and for q4_1 (block sums
-// and min apart) round further than per-element sums.
-//  - One workgroup of 8 waves per CU owns consecutive tiles of 16 rows; the
-//    tiles' units (16 rows x 128 k) are split into equal consecutive runs, one
-//    per wave, kDepth units in flight. Tiles that a wave covers whole it stores
-//    itself, shared ones go through LDS and are added in wave order
-//    (deterministic). x goes to LDS once per workgroup as it is, one barrier.
-//    (16 waves: 19.2 us against 18.5 for 18944 x 3584 q8_0; one unit in flight
-//    21.7, three 19.1.)
-//  - A lane's weight row is lane % 16 and its quarter of each GGUF block (8
-//    elements) lane / 16, for the loads, the decode and the products alike.
-//  - 3..8 rows: v_mfma_f32_4x4x1_16b_f32, exact products and fp32 sums, whose 16
-//    blocks are four rows of x against four weight rows each, the four quarters in
-//    different blocks; a lane's accumulators are the rows of x. (16 x 16 x 4 would
-//    do four times the work for four rows.) One or two rows: fp32 FMA (one row
-//    15.8 us against 21.3 on the MFMA).
-//  - Sums: chains of 16 products, two added per unit, units in order, then the
-//    four quarters. Relative error against 64 bits, K = 3584 1.2e-7, 18944 1.3e-7.
-// Bound by VALU: two to three instructions a weight to make the fp32 values, one
-// more per row; the row-strided 12-byte loads cost ~18 address cycles each. 18944 x
-// 3584, one row: q4_0 15.6 us, q8_0 19.4.
+// (src/cuda_quant.cu:300-361), behind mlq_linear_aos. The kernel here takes one
+// and two rows on few weight tiles; aos_tiles.hip the rest (launch_aos_gemv).
+//  - A workgroup of 8 waves owns 8 output rows (one per wave) and stages x
+//    [m][k] in LDS once (coalesced; 32 elements per block padded to 36
+//    floats so lanes reading consecutive blocks hit different banks).
+//  - A wave walks its row in chunks of 64 blocks. A chunk's bytes (64 x 34 /
+//    18 / 20) are covered by 16-byte units loaded straight into the wave's
+//    LDS area with buffer_load ... lds (no registers), the next chunk in
+//    flight while the current one is used. The row's buffer range starts at
+//    the 16-byte boundary below the row and ends at the 4-byte boundary past
+//    it, so the loads stay inside the pages the row occupies and anything
+//    past the row reads as zero.
+//  - Lane l takes block l of the chunk: its scale(s) with 16-bit reads, its
+//    codes with aligned 32-bit reads funnel-shifted by the block's 2-byte
+//    offset (34- and 18-byte blocks alternate between 4-byte phases).
+//  - Per element (d * q [+ m]) * x in fp32, the reference's per-element
+//    dequant (src/quant.cc:477-503), accumulated per lane in block order;
+//    the lanes' sums are added across the wave at the end.
 #include <hip/hip_runtime.h>
-
-#include <algorithm>
 
 #include "../mlq_layout.h"
 #include "device_common.h"
@@ -41,307 +29,157 @@
 namespace mlq {
 namespace {
 
-constexpr int kWaves = 8;
-constexpr int kDepth = 2;                 // units in flight per wave
-constexpr uint32_t kPast = 0x80000000u;   // an offset past every buffer
+constexpr int kAosWaves = 8;
+constexpr int kAosThreads = 64 * kAosWaves;
+constexpr int kAosChunk = 64;                 // blocks per chunk (one per lane)
+constexpr int kAosBuf = 3 * 1024;             // three 1 KiB DMA loads per chunk
+constexpr int kXBlockFloats = 36;             // 32 elements + pad per block in LDS
 
 struct AosArgs {
-  const uint8_t* w;  // GGUF blocks, row n at w + n * row_bytes
-  const float* x;    // [m][k]
-  float* y;          // [m][n]
-  int m, n, k, nb, g;
+  const uint8_t* w;   // AoS blocks, row n at w + n * row_bytes
+  const float* x;     // [m][k]
+  float* y;           // [m][n]
+  int n, k, nb, m;
   int row_bytes;
-  int tiles, extra;  // tiles per workgroup; the first `extra` have one more
 };
 
 template <int QT>
-__device__ __host__ constexpr int aos_block_bytes() {
+constexpr int aos_block_bytes() {
   return QT == MLQ_Q8_0 ? 34 : QT == MLQ_Q4_0 ? 18 : 20;
 }
 
-// A lane reads, of each of the unit's four blocks, a window from the 4-byte
-// boundary at or below the block (q8_0: plus 8 quarter, q4: plus 8 (quarter %
-// 2)): its 8 code bytes lie 2 or 4 bytes behind the block's phase in it, and in
-// quarter 0 (q4: also 2) the scale (and min) ahead of them. Windows of 12 bytes
-// where every row and the base start on 4-byte boundaries (FOUR: the phase of
-// block b is then known), else of 16; what passes the 4-byte boundary behind the
-// workgroup's rows reads as zero.
-struct Unit {
-  uint4 v[4];
-};
+__device__ __forceinline__ uint32_t lds_u32(const uint8_t* p) { return *(const uint32_t*)p; }
+__device__ __forceinline__ float lds_f16(const uint8_t* p) {
+  return half_bits_to_float(*(const uint16_t*)p);
+}
 
-// 8 code bytes (q4: already one nibble each) -> q (q4_0: q - 8) in fp32, exact.
-template <int QT>
-__device__ __forceinline__ void codes_f32(uint32_t c0, uint32_t c1, float (&q)[8]) {
-  if constexpr (QT == MLQ_Q4_0) {  // n - 8 as a signed byte
-    c0 = (c0 + 0x78787878u) ^ 0x80808080u;
-    c1 = (c1 + 0x78787878u) ^ 0x80808080u;
-  }
+// Four consecutive code words (16 bytes) starting at 2-byte aligned LDS
+// offset `at`.
+__device__ __forceinline__ void code_words(const uint8_t* buf, int at, uint32_t (&w)[8], int nw) {
+  const int a0 = at & ~3;
+  const uint32_t sh = (uint32_t)(at & 3) * 8;
+  uint32_t prev = lds_u32(buf + a0);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const uint32_t b = (j < 4 ? c0 : c1) >> (8 * (j & 3));
-    q[j] = QT == MLQ_Q4_1 ? (float)(uint8_t)b : (float)(int8_t)b;
+  for (int i = 0; i < 8; ++i) {
+    if (i < nw) {
+      const uint32_t next = lds_u32(buf + a0 + 4 * (i + 1));
+      w[i] = sh ? __builtin_amdgcn_alignbit(next, prev, sh) : prev;
+      prev = next;
+    }
   }
 }
 
-template <int QT, int MR, bool FOUR>
-__global__ __launch_bounds__(64 * kWaves) void aos_gemv_kernel(AosArgs a) {
-  constexpr int W = kWaves, BS = aos_block_bytes<QT>();
-  constexpr int NA = MR == 8 ? 2 : 1;     // accumulator quads (4 rows of x each)
-  constexpr int XR = MR < 4 ? MR : 4;     // rows of x of a quad that exist
-  constexpr int kPartTile = 64 * NA;      // (rows past XR are never written nor stored)
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  f4_t* xs = (f4_t*)smem;                 // [k / 4][MR], four columns each
-  // at the end: two partial tiles per wave, [row of x][weight row]
-  float* part = (float*)(xs + a.g * (kGroupK / 4) * MR);
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = a.g;
+template <int QT, int MR>
+__global__ __launch_bounds__(kAosThreads) void aos_gemv_kernel(AosArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  constexpr int BS = aos_block_bytes<QT>();
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int xstride = a.nb * kXBlockFloats;  // floats per row of x in LDS
+  float* xs = (float*)lds;
+  uint8_t* wbuf = lds + (((size_t)MR * xstride * 4 + 255) & ~(size_t)255) +
+                  (size_t)wave * 2 * kAosBuf;
 
-  // this workgroup's tiles and this wave's run of their units
-  const int T = a.tiles + ((int)blockIdx.x < a.extra ? 1 : 0);
-  const int t0 = (int)blockIdx.x * a.tiles + min((int)blockIdx.x, a.extra);
-  const int U = T * G;
-  const int u0 = wave * U / W, u1 = (wave + 1) * U / W, n = u1 - u0;
-  const int first = wave * T / W;  // = u0 / G
-  const int rows0 = t0 * kTileRows;
-  const uint8_t* base = a.w + (size_t)rows0 * a.row_bytes;
-  const int lead = FOUR ? 0 : (int)((uintptr_t)base & 3);
-  const rsrc_t rw = make_rsrc(
-      base - lead,
-      (uint32_t)((lead + (size_t)min(T * kTileRows, a.n - rows0) * a.row_bytes + 3) & ~(size_t)3));
-  const uint32_t arow = (uint32_t)(lead + (lane & 15) * a.row_bytes);
-  const uint32_t aq = QT == MLQ_Q8_0 ? 8u * (lane >> 4) : 8u * ((lane >> 4) & 1);
-
-  int ltile = first, lg = u0 - first * G;  // the next unit to load
-  auto load = [&](Unit& s) __attribute__((always_inline)) {
-    const uint32_t su = (uint32_t)(ltile * kTileRows * a.row_bytes + lg * (kGroupBlocks * BS));
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const uint32_t at = arow + (uint32_t)(b * BS);
-      const int off = (int)((at & ~3u) + aq);
-      if constexpr (FOUR) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b96(rw, off, (int)su, 0);
-        s.v[b] = make_uint4(v[0], v[1], v[2], 0u);
-      } else {
-        s.v[b] = buf_load16(rw, (uint32_t)off, su);
-      }
-    }
-    if (++lg == G) {
-      lg = 0;
-      ++ltile;
-    }
-  };
-  // block b of a unit of group g as fp32 weights
-  auto weights = [&](const Unit& s, int b, int g, float (&w)[8]) __attribute__((always_inline)) {
-    uint4 v = s.v[b];
-    uint32_t head, c0, c1;  // the block's first bytes (scale, min); the lane's codes
-    if constexpr (FOUR) {
-      const bool odd = QT != MLQ_Q4_1 && (b & 1) != 0;  // 34 b and 18 b bytes: phase 2
-      head = odd ? v.x >> 16 : v.x;
-      if constexpr (QT == MLQ_Q4_1) {
-        c0 = v.y;
-        c1 = v.z;
-      } else {
-        c0 = odd ? v.y : __builtin_amdgcn_alignbit(v.y, v.x, 16);
-        c1 = odd ? v.z : __builtin_amdgcn_alignbit(v.z, v.y, 16);
-      }
-    } else {
-      const uint32_t phase = (arow + (uint32_t)(b * BS)) & 3u;
-      head = __builtin_amdgcn_alignbyte(v.y, v.x, phase);
-      const uint32_t p1 = __builtin_amdgcn_alignbyte(v.z, v.y, phase);
-      const uint32_t p2 = __builtin_amdgcn_alignbyte(v.w, v.z, phase);
-      c0 = QT == MLQ_Q4_1 ? p1 : __builtin_amdgcn_alignbit(p1, head, 16);
-      c1 = QT == MLQ_Q4_1 ? p2 : __builtin_amdgcn_alignbit(p2, p1, 16);
-    }
-    // the scale sits in quarter 0 (q4: and 2): to the row's other quarters
-    float h = xor16_pair(__builtin_bit_cast(float, head)).lo;
-    if constexpr (QT == MLQ_Q8_0) h = xor32_pair(h).lo;
-    const uint32_t bits = __builtin_bit_cast(uint32_t, h);
-    float d = half_bits_to_float((uint16_t)bits);
-    float mn = QT == MLQ_Q4_1 ? half_bits_to_float((uint16_t)(bits >> 16)) : 0.0f;
-    if (g * kGroupBlocks + b >= a.nb) d = mn = 0.0f;  // past the row: the next row's blocks
-    if constexpr (QT != MLQ_Q8_0) {
-      const uint32_t sh = 4u * (uint32_t)(lane >> 5);  // elements 16..31: high nibbles
-      c0 = (c0 >> sh) & 0x0F0F0F0Fu;
-      c1 = (c1 >> sh) & 0x0F0F0F0Fu;
-    }
-    codes_f32<QT>(c0, c1, w);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) w[j] = QT == MLQ_Q4_1 ? __builtin_fmaf(d, w[j], mn) : d * w[j];
-  };
-
-  // ---- x into LDS (zeros past m and past k), requested ahead of the weights
-  const rsrc_t rx = make_rsrc(a.x, (uint32_t)((size_t)a.m * a.k * 4));
-  const bool vec = (a.k & 3) == 0;
-  const int quads = G * (kGroupK / 4);
-  auto load_x = [&](f4_t (&v)[MR], int c) __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < MR; ++r) {
-      const uint32_t off = (uint32_t)(r * a.k + 4 * c) * 4u;
-      if (vec) {
-        v[r] = __builtin_bit_cast(f4_t, buf_load16(rx, r < a.m && 4 * c < a.k ? off : kPast, 0));
-      } else {  // the row's end may fall inside a quad
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          v[r][i] = __builtin_bit_cast(
-              float, buf_load4(rx, r < a.m && 4 * c + i < a.k ? off + 4u * i : kPast, 0));
-      }
-    }
-  };
-  auto store_x = [&](const f4_t (&v)[MR], int c) __attribute__((always_inline)) {
-    if (c >= quads) return;
-#pragma unroll
-    for (int r = 0; r < MR; ++r) xs[c * MR + r] = v[r];
-  };
-  Unit ring[kDepth];
-  f4_t xv[MR];
-  load_x(xv, threadIdx.x);
-  if (n >= kDepth) {
-#pragma unroll
-    for (int i = 0; i < kDepth; ++i) load(ring[i]);
-  } else if (n > 0) {
-    load(ring[0]);
-  }
-  store_x(xv, threadIdx.x);
-  for (int c = 64 * W; c < quads; c += 64 * W) {
-    load_x(xv, c + threadIdx.x);
-    store_x(xv, c + threadIdx.x);
+  // x -> LDS, zero past k and for the rows past m up to MR
+  const int kq = a.nb * 32;
+  for (int i = tid; i < MR * kq; i += kAosThreads) {
+    const int r = i / kq, c = i - r * kq;
+    const float v = r < a.m && c < a.k ? a.x[(size_t)r * a.k + c] : 0.0f;
+    xs[r * xstride + (c >> 5) * kXBlockFloats + (c & 31)] = v;
   }
   __syncthreads();
 
-  // ---- the wave's units
-  f4_t acc[NA], head[NA];  // running; the run's first tile if not whole
+  const int row = blockIdx.x * kAosWaves + wave;
+  if (row >= a.n) return;  // (no barrier below)
+  const uint8_t* rowp = a.w + (size_t)row * a.row_bytes;
+  const int lead = (int)((uintptr_t)rowp & 15);
+  const rsrc_t rw = make_rsrc(rowp - lead, (uint32_t)((lead + a.row_bytes + 3) & ~3));
+  const int chunks = (a.nb + kAosChunk - 1) / kAosChunk;
+
+  // chunk c's 16-byte units [u0, u0 + 138) into buffer slot (c & 1); units
+  // past the row read as zero
+  auto fetch = [&](int c) __attribute__((always_inline)) {
+    const int u0 = (lead + c * kAosChunk * BS) >> 4;
+    uint8_t* dst = wbuf + (c & 1) * kAosBuf;
 #pragma unroll
-  for (int i = 0; i < NA; ++i) acc[i] = head[i] = (f4_t){0.f, 0.f, 0.f, 0.f};
-  const f4_t* xl = xs + 2 * (lane >> 4) * MR + (MR <= 2 ? 0 : lane & 3);
-  int tile = first, g = u0 - first * G;
-  // v[r / 4][r % 4] (row r of x, weight row lane % 16) over the four quarters
-  auto quarters = [&](f4_t (&v)[NA]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < NA; ++i)
-#pragma unroll
-      for (int r = 0; r < XR; ++r) v[i][r] = xor32_sum(xor16_sum(v[i][r]));
-  };
-  // output of row 4 i + lane / 16 of x and weight row lane % 16 of tile t
-  auto store = [&](float v, int i, int t) __attribute__((always_inline)) {
-    const int row = (t0 + t) * kTileRows + (lane & 15), r = 4 * i + (lane >> 4);
-    if (row < a.n && r < a.m) a.y[(size_t)r * a.n + row] = v;
-  };
-  auto flush = [&]() __attribute__((always_inline)) {
-    quarters(acc);
-    if (tile * G >= u0 && (tile + 1) * G <= u1) {
-#pragma unroll
-      for (int i = 0; i < NA; ++i) {
-        const f4_t v = acc[i];
-        const int r = lane >> 4;
-        store(XR == 1 || r == 0 ? v[0] : XR == 2 || r == 1 ? v[1] : r == 2 ? v[2] : v[3], i, tile);
-      }
-    } else {  // (the run's last tile stays in acc)
-#pragma unroll
-      for (int i = 0; i < NA; ++i) head[i] = acc[i];
+    for (int j = 0; j < 3; ++j) {
+      const uint32_t off = (uint32_t)((u0 + 64 * j + lane) * 16);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rw, (__attribute__((address_space(3))) void*)(dst + 1024 * j), 16, off, 0, 0, 0);
     }
-#pragma unroll
-    for (int i = 0; i < NA; ++i) acc[i] = (f4_t){0.f, 0.f, 0.f, 0.f};
   };
-  auto run = [&](const Unit& s) __attribute__((always_inline)) {
-    f4_t c[NA][2];
+
+  float acc[MR];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      float w[8];
-      weights(s, b, g, w);
-      const f4_t* xp = xl + (g * 32 + b * 8) * MR;
+  for (int r = 0; r < MR; ++r) acc[r] = 0.0f;
+
+  fetch(0);
+  for (int c = 0; c < chunks; ++c) {
+    if (c + 1 < chunks) {
+      fetch(c + 1);
+      __builtin_amdgcn_s_waitcnt(0x0F73);  // vmcnt(3): chunk c landed
+    } else {
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int b = c * kAosChunk + lane;
+    if (b < a.nb) {
+      const uint8_t* buf = wbuf + (c & 1) * kAosBuf;
+      const int at = (lead + b * BS) - (((lead + c * kAosChunk * BS) >> 4) << 4);
+      const float d = lds_f16(buf + at);
+      const float* xb = xs + b * kXBlockFloats;
+      if constexpr (QT == MLQ_Q8_0) {
+        uint32_t w[8];
+        code_words(buf, at + 2, w, 8);
 #pragma unroll
-      for (int i = 0; i < NA; ++i) {
-        f4_t& ch = c[i][b >> 1];
-        if ((b & 1) == 0) ch = (f4_t){0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 8; ++i) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if constexpr (MR <= 2) {
+          for (int j = 0; j < 4; ++j) {
+            const float wv = d * (float)(int8_t)(w[i] >> (8 * j));
 #pragma unroll
-            for (int r = 0; r < MR; ++r) {
-              const f4_t x4 = xp[h * MR + r];
-#pragma unroll
-              for (int j = 0; j < 4; ++j) ch[r] = __builtin_fmaf(x4[j], w[4 * h + j], ch[r]);
-            }
-            continue;
+            for (int r = 0; r < MR; ++r) acc[r] = fmaf(wv, xb[r * xstride + 4 * i + j], acc[r]);
           }
-          const f4_t x4 = xp[h * MR + 4 * i];
+        }
+      } else {
+        const float mn = QT == MLQ_Q4_1 ? lds_f16(buf + at + 2) : 0.0f;
+        uint32_t w[8];
+        code_words(buf, at + (QT == MLQ_Q4_1 ? 4 : 2), w, 4);
+        // element e < 16: low nibble of byte e; e >= 16: high nibble of byte e - 16
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            ch = __builtin_amdgcn_mfma_f32_4x4x1f32(x4[j], w[4 * h + j], ch, 0, 0, 0);
+        for (int half = 0; half < 2; ++half) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const int q = (int)((w[i] >> (8 * j + 4 * half)) & 15);
+              const float wv = QT == MLQ_Q4_0 ? d * (float)(q - 8) : d * (float)q + mn;
+              const int e = 16 * half + 4 * i + j;
+#pragma unroll
+              for (int r = 0; r < MR; ++r) acc[r] = fmaf(wv, xb[r * xstride + e], acc[r]);
+            }
+          }
         }
       }
     }
-#pragma unroll
-    for (int i = 0; i < NA; ++i)
-#pragma unroll
-      for (int r = 0; r < XR; ++r) acc[i][r] += c[i][0][r] + c[i][1][r];
-    if (++g == G) {
-      flush();
-      g = 0;
-      ++tile;
-    }
-  };
-  // No load past the run's end: the 16 waves' would cost a microsecond of
-  // address cycles.
-  int j = 0;
-  for (; j + 2 * kDepth <= n; j += kDepth) {
-#pragma unroll
-    for (int i = 0; i < kDepth; ++i) {
-      run(ring[i]);
-      load(ring[i]);
-    }
-  }
-  const int left = n - j;  // fewer than 2 kDepth, kDepth of them loaded
-#pragma unroll
-  for (int i = 0; i < kDepth; ++i) {
-    if (i < left) run(ring[i]);
-    if (i + kDepth < left) load(ring[i]);
+    // this chunk's slot is refilled two chunks later: every lane is done
+    // reading it before the next fetch (issued at the top of the loop)
+    __builtin_amdgcn_wave_barrier();
   }
 #pragma unroll
-  for (int i = 0; i < kDepth; ++i)
-    if (i + kDepth < left) run(ring[i]);
-
-  // ---- partial tiles: a run's first one (head, or acc if the run ends inside
-  // it) in slot 0, its last in slot 1; added in wave order
-  quarters(acc);
-  if (lane < 16) {
-    float* p = part + wave * 2 * kPartTile + lane;
-#pragma unroll
-    for (int i = 0; i < NA; ++i)
-#pragma unroll
-      for (int r = 0; r < XR; ++r) {
-        p[(4 * i + r) * 16] = tile == first ? acc[i][r] : head[i][r];
-        p[kPartTile + (4 * i + r) * 16] = acc[i][r];
-      }
-  }
-  __syncthreads();
-  for (int t = wave; t < T; t += W) {
-    float v[NA];
-#pragma unroll
-    for (int i = 0; i < NA; ++i) v[i] = 0.0f;
-    bool whole = false;  // one wave had all of it and stored it
-    // (over all waves: the reads are in flight together, and finding the first
-    // and last one that met the tile takes two divisions)
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      const int lo = w * U / W, hi = (w + 1) * U / W;
-      const bool met = max(lo, t * G) < min(hi, (t + 1) * G);
-      whole |= lo <= t * G && hi >= (t + 1) * G;
-      const float* p = part + (w * 2 + (lo >= t * G ? 0 : 1)) * kPartTile + lane;
-#pragma unroll
-      for (int i = 0; i < NA; ++i) v[i] += met ? p[64 * i] : 0.0f;
-    }
-    if (!whole) {
-#pragma unroll
-      for (int i = 0; i < NA; ++i) store(v[i], i, t);
-    }
+  for (int r = 0; r < MR; ++r) {
+    const float s = wave_sum(acc[r]);
+    if (lane == 0 && r < a.m) a.y[(size_t)r * a.n + row] = s;
   }
 }
 
 // x rows the kernel holds for m activation rows (MR)
 int aos_rows(int m) { return m == 1 ? 1 : m == 2 ? 2 : m <= 4 ? 4 : 8; }
+
+size_t aos_lds_bytes(int m, int nb) {
+  return (((size_t)aos_rows(m) * nb * kXBlockFloats * 4 + 255) & ~(size_t)255) +
+         (size_t)kAosWaves * 2 * kAosBuf;
+}
 
 size_t aos_lds_limit() {
   static const size_t limit = [] {
@@ -356,64 +194,67 @@ size_t aos_lds_limit() {
   return limit;
 }
 
-template <int QT, int MR, bool FOUR>
-hipError_t launch_mr(const AosArgs& a, int grid, hipStream_t stream) {
-  constexpr size_t kParts = (size_t)kWaves * 2 * 64 * (MR == 8 ? 2 : 1) * sizeof(float);
-  const size_t lds = (size_t)a.g * kGroupK * MR * sizeof(float) + kParts;
-  const auto kernel = aos_gemv_kernel<QT, MR, FOUR>;
-  const hipError_t e = allow_dynamic_lds((const void*)kernel, lds);
+template <int QT, int MR>
+hipError_t launch_mr(const AosArgs& a, size_t lds, hipStream_t stream) {
+  const hipError_t e = allow_dynamic_lds((const void*)aos_gemv_kernel<QT, MR>, lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kWaves), lds, stream, a);
+  const unsigned grid = (unsigned)((a.n + kAosWaves - 1) / kAosWaves);
+  aos_gemv_kernel<QT, MR><<<grid, kAosThreads, lds, stream>>>(a);
   return hipGetLastError();
 }
 
-template <int QT, bool FOUR>
-hipError_t launch_rows_of(const AosArgs& a, int grid, hipStream_t stream) {
-  if (a.m == 1) return launch_mr<QT, 1, FOUR>(a, grid, stream);
-  if (a.m == 2) return launch_mr<QT, 2, FOUR>(a, grid, stream);
-  if (a.m <= 4) return launch_mr<QT, 4, FOUR>(a, grid, stream);
-  return launch_mr<QT, 8, FOUR>(a, grid, stream);
-}
-
 template <int QT>
-hipError_t launch_typed(const AosArgs& a, int grid, hipStream_t stream) {
-  const bool four = ((uintptr_t)a.w & 3) == 0 && a.row_bytes % 4 == 0;
-  return four ? launch_rows_of<QT, true>(a, grid, stream)
-              : launch_rows_of<QT, false>(a, grid, stream);
+hipError_t launch_typed(const AosArgs& a, size_t lds, hipStream_t stream) {
+  return a.m == 1 ? launch_mr<QT, 1>(a, lds, stream) : launch_mr<QT, 2>(a, lds, stream);
 }
 
 }  // namespace
 
-// The row counts and lengths that need no workspace: rows of x padded to 1, 2, 4
-// or 8, at 144 bytes per 32 elements, beside 48 KiB. (x takes 128 of them, up to a
-// 128-k group more, and the partial tiles 8 KiB.)
+// The row counts and lengths that need no workspace: what the kernel above
+// stages, of which the one for many tiles needs less (128 bytes per 32 elements
+// and row, up to a 128-k group more, and 8 KiB).
 bool aos_gemv_supported(int type, int m, int n, int k) {
   if (m < 1 || m > 8 || n < 1 || k < 1) return false;
   if (type != MLQ_Q8_0 && type != MLQ_Q4_0 && type != MLQ_Q4_1) return false;
-  const size_t nb = (size_t)((k + kQK - 1) / kQK);
-  return (((size_t)aos_rows(m) * nb * 144 + 255) & ~(size_t)255) + 48 * 1024 <= aos_lds_limit();
+  const int nb = (k + kQK - 1) / kQK;
+  return aos_lds_bytes(m, nb) <= aos_lds_limit();
+}
+
+// One and two rows on few tiles: this kernel's 8-row workgroups start faster and
+// fill more CUs than a workgroup per 16-row tile. Both measured over K 512..14336
+// and 256..16384 weight rows (us, this kernel against aos_tiles.hip's, q4_0, q8_0 much
+// the same): one row on at most half a tile per CU 1.07 to 1.6 times faster (2048 x
+// 4096 5.0, 7.6), up to 1.5 tiles and K 4096 from 0.85 to 1.3 with how K fits the
+// 2048-k chunks (4096 x 4096 of q8_0 8.2, 8.4; x 2048 4.5, 5.5; x 3584 6.9, 6.3),
+// past either line slower (8192 x 2048 8.2, 7.9; 4096 x 8192 17.9, 12.3); two rows
+// on at most half a tile per CU 0.8 to 1.35 (2048 x 4096 6.8, 8.4; 3072 x 4096
+// 12.7, 8.8). (A base off 2-byte boundaries would put its 16-bit LDS reads there.)
+bool few_tiles(const void* aos, int m, int nt, int k) {
+  if (m > 2 || ((uintptr_t)aos & 1) != 0) return false;
+  const int cus = device_cus();
+  return 2 * nt <= cus || (m == 1 && 2 * nt <= 3 * cus && k <= 4096);
 }
 
 hipError_t launch_aos_gemv(int type, const void* aos, int n, int k, const float* x, float* y,
                            int m, hipStream_t stream) {
   if (!aos_gemv_supported(type, m, n, k) || ((uintptr_t)aos & 1) != 0) return hipErrorInvalidValue;
-  const Geometry geo = geometry(n, k);
-  const int grid = std::min(geo.nt, device_cus());
-  AosArgs a = {};
+  if (!few_tiles(aos, m, geometry(n, k).nt, k))
+    return launch_aos_tiles(type, aos, n, k, x, y, m, stream);
+  AosArgs a;
   a.w = (const uint8_t*)aos;
   a.x = x;
   a.y = y;
-  a.m = m;
   a.n = n;
   a.k = k;
-  a.nb = geo.nb;
-  a.g = geo.g;
-  a.tiles = geo.nt / grid;
-  a.extra = geo.nt % grid;
+  a.nb = (k + kQK - 1) / kQK;
+  a.m = m;
+  const int bs = type == MLQ_Q8_0 ? 34 : type == MLQ_Q4_0 ? 18 : 20;
+  a.row_bytes = a.nb * bs;
+  const size_t lds = aos_lds_bytes(m, a.nb);
   switch (type) {
-    case MLQ_Q8_0: a.row_bytes = geo.nb * 34; return launch_typed<MLQ_Q8_0>(a, grid, stream);
-    case MLQ_Q4_0: a.row_bytes = geo.nb * 18; return launch_typed<MLQ_Q4_0>(a, grid, stream);
-    default: a.row_bytes = geo.nb * 20; return launch_typed<MLQ_Q4_1>(a, grid, stream);
+    case MLQ_Q8_0: return launch_typed<MLQ_Q8_0>(a, lds, stream);
+    case MLQ_Q4_0: return launch_typed<MLQ_Q4_0>(a, lds, stream);
+    default: return launch_typed<MLQ_Q4_1>(a, lds, stream);
   }
 }
 

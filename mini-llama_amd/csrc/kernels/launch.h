@@ -172,9 +172,12 @@ bool skinny_plan_set();
 
 // aos_gemv.hip: GEMV straight from GGUF AoS blocks (m <= 8 rows of x, x
 // staged in LDS: aos_gemv_supported says whether the shape fits).
+// launch_aos_tiles (aos_tiles.hip): its kernel for many weight tiles or rows.
 bool aos_gemv_supported(int type, int m, int n, int k);
 hipError_t launch_aos_gemv(int type, const void* aos, int n, int k, const float* x, float* y,
                            int m, hipStream_t stream);
+hipError_t launch_aos_tiles(int type, const void* aos, int n, int k, const float* x, float* y,
+                            int m, hipStream_t stream);
 
 // linear_f32.hip: fp32 W [n][k], any m (passes of up to 8 rows).
 hipError_t launch_linear_f32(const float* w, int n, int k, const float* x, float* y, int m,

@@ -786,12 +786,13 @@ def test_resident_rows(pkg, cuda, qtype, m, n, k):
         assert bool(((y - torch.nn.functional.silu(gate) * up).abs() <= slack).all())
 
 
-# Raw GGUF blocks with several tiles per workgroup (whole and shared ones), odd block counts (rows off
+# Raw GGUF blocks on both sides of the lines between their two kernels, several tiles per workgroup (whole and shared), odd block counts (rows off
 # 4-byte boundaries), k % 4 != 0, a base off a 4-byte boundary, blocks of the last group past the row.
 @pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("m,n,k", [(1, 9001, 1056), (3, 8200, 3104), (8, 4500, 994), (1, 20000, 99), (2, 16411, 128),
                                    # one row of 1, 33 and 65 groups
-                                   (1, 64, 96), (1, 64, 4224), (1, 4112, 8320)])
+                                   (1, 64, 96), (1, 64, 4224), (1, 4112, 8320),
+                                   (1, 2048, 4128), (1, 2064, 4128), (1, 6144, 4096), (1, 6160, 4096), (2, 2048, 96), (2, 2064, 96)])
 def test_aos_many_tiles(pkg, cuda, qtype, m, n, k):
     import torch
     from synthetic import synth
