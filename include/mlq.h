@@ -268,7 +268,7 @@ int mlq_gguf_upload(const mlq_gguf* g, int64_t index, void* aos_dev, size_t aos_
  * (src/cuda_quant.cu:300-361). Up to 8 rows of x whose k fits the kernel's
  * LDS staging (mlq_linear_aos_workspace reports 0 bytes) run a GEMV that
  * reads the blocks as they are, every weight byte once; `workspace` may
- * then be NULL. aos_dev is 2-byte aligned, as the blocks are. Otherwise the blocks are repacked into `workspace` (device,
+ * then be NULL. Otherwise the blocks are repacked into `workspace` (device,
  * >= mlq_weight_layout(...).bytes) and run through mlq_linear. Results
  * meet the Linear's tolerance either way (the direct GEMV dequantizes and sums
  * in fp32 like the reference's per-element loop, in another order). */

@@ -237,7 +237,7 @@ bool few_tiles(const void* aos, int m, int nt, int k) {
 
 hipError_t launch_aos_gemv(int type, const void* aos, int n, int k, const float* x, float* y,
                            int m, hipStream_t stream) {
-  if (!aos_gemv_supported(type, m, n, k) || ((uintptr_t)aos & 1) != 0) return hipErrorInvalidValue;
+  if (!aos_gemv_supported(type, m, n, k)) return hipErrorInvalidValue;
   if (!few_tiles(aos, m, geometry(n, k).nt, k))
     return launch_aos_tiles(type, aos, n, k, x, y, m, stream);
   AosArgs a;

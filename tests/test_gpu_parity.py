@@ -804,7 +804,7 @@ def test_aos_many_tiles(pkg, cuda, qtype, m, n, k):
     ref = x64 @ w64.t().contiguous()
     # x to 2^-22, fp32 sums
     bound = 2.0 ** -20 * (x64.abs() @ w64.abs().t().contiguous())
-    for lead in (0, 2):
+    for lead in (0, 1, 2, 3):  # blocks at any byte
         buf = torch.zeros(raw.numel() + 16, dtype=torch.uint8, device=cuda)
         buf[lead:lead + raw.numel()] = raw
         y = pkg.linear_aos(qtype, buf[lead:lead + raw.numel()], n, k, x).view(m, n).double()
