@@ -803,30 +803,35 @@ __global__ __launch_bounds__(kAttnRegWaves * 64) void attn_reg_kernel(AttnArgs a
 // j + 16k, D[4*(l/16) + r][l % 16] in register r of lane l.
 __host__ __device__ constexpr int prefill_waves(int hd) { return hd == 256 ? 2 : 4; }
 
-template <int HD, int GP>
-__global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(AttnArgs a) {
+template <int HD>
+constexpr int prefill_lds_floats() {  // K chunk + P per wave; at the end the waves' partials
+  constexpr int W = prefill_waves(HD), slab = 16 * (HD + 4) + 16 * 20;
+  constexpr int merge = W * (16 * (HD + 4) + 32);
+  return W * slab > merge ? W * slab : merge;
+}
+
+// tile: 16 / GP query rows from row tile * 16 / GP on; lds: prefill_lds_floats.
+// AHEAD: the next keys' rows in flight (a hundred registers).
+template <int HD, int GP, bool AHEAD>
+__device__ __forceinline__ void prefill_tile(const AttnArgs& a, int tile, int kvh, float* lds) {
   constexpr int W = prefill_waves(HD);
   constexpr int QT = 16 / GP;   // query rows per tile
   constexpr int KC = 16;        // keys per chunk
   constexpr int NT = HD / 16;   // output tiles
   constexpr int KS = HD + 4;    // padded LDS row of K (16-byte aligned)
   constexpr int KF4 = KC * HD / 4 / 64;  // float4 of a K chunk per lane
-  constexpr bool VPRE = HD <= 128;       // V of the next chunk loaded ahead
+  constexpr bool VPRE = AHEAD && HD <= 128;  // V of the next chunk loaded ahead
   // LDS row strides chosen so the 64 lanes of a wave hit distinct banks:
   // P rows 4q + i (q = lane / 16) start 16 banks apart (20 floats), merge
   // rows likewise (HD + 4)
   constexpr int PS = 20;                           // P row stride (floats)
   constexpr int MS = HD + 4;                       // merge row stride (floats)
   constexpr int SLAB = KC * KS + 16 * PS;          // per wave: K chunk + P
-  constexpr int MERGE = W * (16 * MS + 32);        // partial acc + max / sum
-  constexpr int LDSF = W * SLAB > MERGE ? W * SLAB : MERGE;
-  __shared__ __align__(16) float lds[LDSF];
 
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const int kvh = blockIdx.y;
   const int G = a.group;
-  const int r0 = blockIdx.x * QT;  // first query row of the tile
+  const int r0 = tile * QT;  // first query row of the tile
   const int pos0 = a.pos;
   const int last_row = min(r0 + QT, a.rows) - 1;
   const int kmax = pos0 + last_row;  // last key any row of the tile sees
@@ -896,12 +901,13 @@ __global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(At
   };
   f4_t kn[KF4];
   float vn[VPRE ? NT * 4 : 1];
-  if (wave < nchunks) {
+  if (AHEAD && wave < nchunks) {
     load_k(wave * KC, kn);
     if constexpr (VPRE) load_v(wave * KC, vn);
   }
   for (int c = wave; c < nchunks; c += W) {
     const int k0 = c * KC;
+    if constexpr (!AHEAD) load_k(k0, kn);
 #pragma unroll
     for (int u = 0; u < KF4; ++u) {
       const int f = lane + 64 * u;
@@ -914,7 +920,7 @@ __global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(At
 #pragma unroll
       for (int e = 0; e < NT * 4; ++e) vc[e] = vn[e];
     }
-    if (c + W < nchunks) {
+    if (AHEAD && c + W < nchunks) {
       load_k(k0 + W * KC, kn);
       if constexpr (VPRE) load_v(k0 + W * KC, vn);
     }
@@ -1014,13 +1020,22 @@ __global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(At
   }
 }
 
-// ---- prefill attention, many rows: fp16 pairs on v_mfma_f32_32x32x16_f16 ---------------
+template <int HD, int GP>
+__global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(AttnArgs a) {
+  __shared__ __align__(16) float lds[prefill_lds_floats<HD>()];
+  prefill_tile<HD, GP, true>(a, blockIdx.x, blockIdx.y, lds);
+}
+
+// ---- prefill attention, many rows: bf16 triples on v_mfma_f32_32x32x16_bf16 -------------
 // The kernel above is bound by the fp32 matrix rate (57 TFLOP/s of the causal
-// products at 2000 tokens, 28 heads on 4: 498 us, this one 182). Here
-// every operand is split into two fp16 values, x = hi + lo to 2^-23 of x (its
-// row first scaled by a power of two into fp16's range), and a product is
-// hi hi + hi lo + lo hi (the dropped lo lo is below 2^-24 of it): three
-// products at sixteen times the rate.
+// products at 2000 tokens, 28 heads on 4: 444 us, this one 223). Here every
+// operand is split into three bf16 values, x = hi + mid + lo exactly (8 bits
+// each, with fp32's exponents: no scales, so a row's result depends on nothing but
+// what it sees), and a product is its six largest part products; the three dropped
+// are below 2^-25 of it. Six products at sixteen times the rate. Error against 64
+// bits 0.6 of the fp32 tiles' (normal inputs, per row and head: 2000 tokens 1.9e-7,
+// 3.5e-7; 512 after 1500 2.2e-7, 4.3e-7). fp16 pairs under a scale per four keys
+// take 182 us, but lose values far below their neighbours', masked ones included.
 //  - A workgroup owns 128 (query row, head) pairs of one kv head, a wave 32 of
 //    them as the columns of both products, S^T = K Q^T and O^T = V^T P^T. A
 //    lane then holds 16 keys of one column, so the softmax over keys is in
@@ -1028,45 +1043,76 @@ __global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(At
 //    second product: its k slots take the keys in the order the first one
 //    leaves them, and V^T is stored in that order.
 //  - Tiles of 32 keys: each thread splits 4 keys x 4 dims of K and of V into
-//    LDS (V transposed in registers), double buffered, the next tile's rows
-//    in flight; one barrier per tile.
-//  - Scales: K per four keys (applied to the scores), Q per row, V per four keys, folded
-//    into P relative to the largest seen (the accumulators are rescaled when
-//    that grows); P itself is kept times 2^14, so its low half stays above
-//    fp16's subnormals.
+//    LDS (V transposed in registers), V's rows in flight during the scores, the
+//    next K's during the output.
+//  - Few roundings at a result's own size: small part products first, two
+//    accumulators for a score's large ones, a tile's output summed from zero.
+//  - Two workgroups per CU, up to 256 registers a wave: no branch around a
+//    tile's work (a wave whose rows end before the last tiles adds zeros: the
+//    second copy of the loop's values spilled).
+//  - Values that the split or the products of a masked weight (0) do not carry,
+//    infinite, NaN or from 2^127 on: a workgroup that met one computes its rows
+//    again with the fp32 tiles, so they give what those give.
 //  - Workgroups with the most keys start first; the kv head is the fastest
 //    grid index, so with 4 or 8 of them an XCD's L2 serves one or two.
-constexpr int kPairRows = 128, kPairKeys = 32;
+constexpr int kSplitRows = 128, kSplitKeys = 32;
+typedef __bf16 b2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 b4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 b8_t __attribute__((ext_vector_type(8)));
+
 template <int HD>
-struct PairTile {
-  _Float16 k[2][kPairKeys][HD + 8];   // hi, lo: [key][dim]
-  _Float16 v[2][HD][kPairKeys + 8];   // hi, lo: [dim][key slot], see v_unit
-  float ks[kPairKeys / 4], vs[kPairKeys / 4];  // 2^-e of four keys' K and V
+struct SplitTile {
+  __bf16 k[3][kSplitKeys][HD + 8];   // hi, mid, lo: [key][dim]
+  __bf16 v[3][HD][kSplitKeys + 8];   // hi, mid, lo: [dim][key slot], see v_unit
+  // lo of q's first steps per wave and lane (in registers they spill)
+  static constexpr int kQSteps = HD == 128 ? 4 : 0;
+  b8_t q[kQSteps > 0 ? kQSteps : 1][4][64];
 };
+template <int HD>
+constexpr size_t split_lds_bytes() {
+  constexpr size_t tile = sizeof(SplitTile<HD>), again = prefill_lds_floats<HD>() * sizeof(float);
+  return tile > again ? tile : again;
+}
 
 // Where the 8-slot unit of a dim's row lies: a thread writes four dims of four
 // keys, so neighbouring lanes are four rows (16 banks) apart; turning the
 // units by the dim spreads 16 of them over the banks.
 __device__ __forceinline__ int v_unit(int unit, int dim) { return (unit ^ ((dim >> 4) & 3)) * 8; }
-__device__ __forceinline__ uint2 pack4(_Float16 a, _Float16 b, _Float16 c, _Float16 d) {
-  return make_uint2(as_u32(h2_t{a, b}), as_u32(h2_t{c, d}));
+
+// a, b = p[0] + p[1] + p[2]
+__device__ __forceinline__ void split3(float a, float b, b2_t (&p)[3]) {
+  f2_t x = {a, b};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    p[i] = __builtin_convertvector(x, b2_t);
+    if (i < 2) {
+      x.x -= (float)p[i].x;
+      x.y -= (float)p[i].y;
+    }
+  }
+}
+__device__ __forceinline__ float abs_maximum_f4(float m, f4_t v) {
+  m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(v.x)),
+                                    __builtin_fabsf(v.y));
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(v.z)),
+                                       __builtin_fabsf(v.w));
 }
 
 template <int HD, int GP>
-__global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, 2) void attn_split_kernel(AttnArgs a) {
   constexpr int KT = HD / 16;   // 16-dim steps of the scores
   constexpr int VB = HD / 32;   // 32-dim blocks of the output
   constexpr int DG = HD / 4;    // threads across a key's dims
-  extern __shared__ __align__(16) uint8_t pair_smem[];
-  PairTile<HD>* tiles = (PairTile<HD>*)pair_smem;
+  extern __shared__ __align__(16) uint8_t split_smem[];
+  SplitTile<HD>& tl = *(SplitTile<HD>*)split_smem;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, half = lane >> 5;
   const int G = a.group;
   const int kvh = blockIdx.x % a.n_kv;
-  const int r0 = ((int)(gridDim.x / a.n_kv) - 1 - (int)(blockIdx.x / a.n_kv)) * (kPairRows / GP);
-  const int kmax = a.pos + min(r0 + kPairRows / GP, a.rows) - 1;  // last key any row sees
-  const int nt = kmax / kPairKeys + 1;
+  const int r0 = ((int)(gridDim.x / a.n_kv) - 1 - (int)(blockIdx.x / a.n_kv)) * (kSplitRows / GP);
+  const int kmax = a.pos + min(r0 + kSplitRows / GP, a.rows) - 1;  // last key any row sees
+  const int nt = kmax / kSplitKeys + 1;
   const size_t row_stride = (size_t)a.n_kv * HD;
   const size_t cbase = (size_t)a.layer * a.max_seq * row_stride + (size_t)kvh * HD;
   const uint32_t rs4 = (uint32_t)row_stride * 4u;
@@ -1076,58 +1122,43 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
 
   // this thread's piece of a tile: keys 4 kg .. + 3, dims 4 dg .. + 3
   const int dg = tid % DG, kg = tid / DG;
-  const bool loads = kg < kPairKeys / 4;  // (HD 64: half of the threads)
-  f4_t kr[4], vr[4];
-  auto load = [&](int t) __attribute__((always_inline)) {
-    const uint32_t off = loads ? (uint32_t)(t * kPairKeys + 4 * kg) * rs4 + 16u * dg : 0x80000000u;
+  const bool loads = kg < kSplitKeys / 4;  // (HD 64: half of the threads)
+  f4_t x4[4];            // of K or V: whichever is split next
+  float largest = 0.0f;  // |x| of what this thread reads; NaN stays
+  auto load = [&](rsrc_t r, int t) __attribute__((always_inline)) {
+    const uint32_t off = loads ? (uint32_t)(t * kSplitKeys + 4 * kg) * rs4 + 16u * dg : 0x80000000u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x4[i] = __builtin_bit_cast(f4_t, buf_load16(r, off + i * rs4, 0));
+  };
+  auto split_k = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) largest = abs_maximum_f4(largest, x4[i]);
+    if (!loads) return;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      kr[i] = __builtin_bit_cast(f4_t, buf_load16(rk, off + i * rs4, 0));
-      vr[i] = __builtin_bit_cast(f4_t, buf_load16(rv, off + i * rs4, 0));
+      b2_t x[3], y[3];
+      split3(x4[i].x, x4[i].y, x);
+      split3(x4[i].z, x4[i].w, y);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        *(b4_t*)&tl.k[q][4 * kg + i][4 * dg] = b4_t{x[q].x, x[q].y, y[q].x, y[q].y};
     }
   };
-  auto amax = [&](const f4_t (&r)[4]) __attribute__((always_inline)) {
-    float mx = 0.0f;
+  auto split_v = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      mx = fmaxf(fmaxf(fmaxf(mx, fabsf(r[i].x)), fmaxf(fabsf(r[i].y), fabsf(r[i].z))), fabsf(r[i].w));
-    return row_max<DG>(mx);
-  };
-  auto split = [&](PairTile<HD>& t) __attribute__((always_inline)) {
+    for (int i = 0; i < 4; ++i) largest = abs_maximum_f4(largest, x4[i]);
+    if (!loads) return;
     // slot of the key group in a 16-key run: keys 0-3, 8-11 | 4-7, 12-15
     const int unit = 2 * (kg >> 2) + (kg & 1), sub = 4 * ((kg >> 1) & 1);
-    const float ka = amax(kr), va = amax(vr);
-    const int ke = min(pow2_scale_exp(ka), 126), ve = min(pow2_scale_exp(va), 126);
-    const float kf = ldexp_f(1.0f, ke), vf = ldexp_f(1.0f, ve);
-    if (!loads) return;
-    if (dg == 0) {
-      t.ks[kg] = ldexp_f(1.0f, -ke);
-      t.vs[kg] = va == 0.0f ? 0.0f : ldexp_f(1.0f, -ve);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      _Float16 h[4], l[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float x = kr[i][j] * kf;
-        h[j] = (_Float16)x;
-        l[j] = (_Float16)(x - (float)h[j]);
-      }
-      *(uint2*)&t.k[0][4 * kg + i][4 * dg] = pack4(h[0], h[1], h[2], h[3]);
-      *(uint2*)&t.k[1][4 * kg + i][4 * dg] = pack4(l[0], l[1], l[2], l[3]);
-    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // dim 4 dg + j of the four keys
-      _Float16 h[4], l[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float y = vr[i][j] * vf;
-        h[i] = (_Float16)y;
-        l[i] = (_Float16)(y - (float)h[i]);
-      }
+      b2_t x[3], y[3];
+      split3(x4[0][j], x4[1][j], x);
+      split3(x4[2][j], x4[3][j], y);
       const int dim = 4 * dg + j, at = v_unit(unit, dim) + sub;
-      *(uint2*)&t.v[0][dim][at] = pack4(h[0], h[1], h[2], h[3]);
-      *(uint2*)&t.v[1][dim][at] = pack4(l[0], l[1], l[2], l[3]);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        *(b4_t*)&tl.v[q][dim][at] = b4_t{x[q].x, x[q].y, y[q].x, y[q].y};
     }
   };
 
@@ -1136,35 +1167,33 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   const int qr = r0 + (c0 + col) / GP, qh = (c0 + col) % GP;
   const bool live = qr < a.rows && qh < G;
   const int qpos = a.pos + qr;
-  const int wmin = a.pos + r0 + c0 / GP;  // the first and last key the wave's rows see
-  const int wmax = min(a.pos + r0 + (c0 + 31) / GP, kmax);
-  h8_t qhi[KT], qlo[KT];
-  float qscale;
+  const int wmin = a.pos + r0 + c0 / GP;  // the last key the wave's first row sees
+  // softmax in base 2: scores times scale log2(e)
+  const float sl2 = a.scale * 1.44269504088896341f;
+  constexpr int QL = SplitTile<HD>::kQSteps;
+  b8_t q[3][KT];  // (the first QL of q[2] in LDS)
   {
     const float* qp = a.q + (size_t)(live ? qr : 0) * a.q_stride +
                       (size_t)(kvh * G + (live ? qh : 0)) * HD + 8 * half;
-    f4_t x[KT][2];
-    float mx = 0.0f;
 #pragma unroll
     for (int s = 0; s < KT; ++s)
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        x[s][u] = live ? *(const f4_t*)(qp + 16 * s + 4 * u) : f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        const f4_t x = live ? *(const f4_t*)(qp + 16 * s + 4 * u) : f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        largest = abs_maximum_f4(largest, x);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, fabsf(x[s][u][j]));
+        for (int j = 0; j < 2; ++j) {
+          b2_t p[3];
+          split3(x[2 * j], x[2 * j + 1], p);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            q[i][s][4 * u + 2 * j] = p[i].x;
+            q[i][s][4 * u + 2 * j + 1] = p[i].y;
+          }
+        }
       }
-    const int e = min(pow2_scale_exp(xor32_max(mx)), 126);
-    const float f = ldexp_f(1.0f, e);
-    // softmax in base 2: scores times scale log2(e)
-    qscale = a.scale * 1.44269504088896341f * ldexp_f(1.0f, -e);
 #pragma unroll
-    for (int s = 0; s < KT; ++s)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float v = x[s][j >> 2][j & 3] * f;
-        qhi[s][j] = (_Float16)v;
-        qlo[s][j] = (_Float16)(v - (float)qhi[s][j]);
-      }
+    for (int s = 0; s < QL; ++s) tl.q[s][wave][lane] = q[2][s];  // (read by this lane only)
   }
 
   typedef float f16v __attribute__((ext_vector_type(16)));
@@ -1172,87 +1201,123 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
 #pragma unroll
   for (int b = 0; b < VB; ++b) acc[b] = (f16v){};
   float m = -INFINITY, l = 0.0f;  // of the column; l of this half's keys
-  float ref = 0.0f;               // largest V scale so far (wave-uniform)
 
-  load(0);
+  load(rk, 0);
   for (int t = 0; t < nt; ++t) {
-    PairTile<HD>& tl = tiles[t & 1];
-    split(tl);
-    if (t + 1 < nt) load(t + 1);
+    const int k0 = t * kSplitKeys;
+    split_k();  // (the last tile's K is done with since its second barrier)
+    load(rv, t);
     __syncthreads();
-    const int k0 = t * kPairKeys;
-    if (k0 > wmax) continue;  // (the wave's rows end before this tile)
     f16v s = {};
+    // the small products of all dims first: only eight roundings at the
+    // score's own size
 #pragma unroll
     for (int i = 0; i < KT; ++i) {
-      const h8_t kh = *(const h8_t*)&tl.k[0][col][16 * i + 8 * half];
-      const h8_t kl = *(const h8_t*)&tl.k[1][col][16 * i + 8 * half];
-      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qhi[i], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qlo[i], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qhi[i], s, 0, 0, 0);
+      const b8_t kh = *(const b8_t*)&tl.k[0][col][16 * i + 8 * half];
+      const b8_t km = *(const b8_t*)&tl.k[1][col][16 * i + 8 * half];
+      const b8_t kl = *(const b8_t*)&tl.k[2][col][16 * i + 8 * half];
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kl, q[0][i], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, i < QL ? tl.q[i][wave][lane] : q[2][i], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(km, q[1][i], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(km, q[0][i], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, q[1][i], s, 0, 0, 0);
     }
+    // (read again: held across the loops, the hi parts spill)
+    asm volatile("" ::: "memory");
+    f16v s1 = {};
+#pragma unroll
+    for (int i = 0; i < KT; ++i) {
+      const b8_t kh = *(const b8_t*)&tl.k[0][col][16 * i + 8 * half];
+      f16v& c = i % 2 == 0 ? s : s1;
+      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, q[0][i], c, 0, 0, 0);
+    }
+    s += s1;
+    split_v();
+    if (t + 1 < nt) load(rk, t + 1);
+    __syncthreads();
     // lane: keys 8 (i / 4) + 4 half + i % 4 of its column
-    float vsc[4], mx = m, vmax = ref;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float ks = tl.ks[2 * q + half] * qscale;
-      vsc[q] = tl.vs[2 * q + half];
-      vmax = fmaxf(vmax, vsc[q]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s[4 * q + j] *= ks;
-    }
-    if (k0 + kPairKeys - 1 > wmin) {  // the causal edge crosses the tile
+    if (k0 + kSplitKeys - 1 > wmin) {  // the causal edge crosses the tile
 #pragma unroll
       for (int i = 0; i < 16; ++i)
         s[i] = k0 + 8 * (i >> 2) + 4 * half + (i & 3) <= qpos ? s[i] : -INFINITY;
     }
+    float mx = s[0];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    mx = xor32_max(mx);
-    vmax = xor32_max(vmax);
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    mx = fmaxf(m, xor32_max(mx) * sl2);
     // rows with nothing visible yet keep m = -inf and weight 0
     const float base = mx == -INFINITY ? 0.0f : mx;
     const float alpha = mx == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mx);
-    const float inv = vmax > 0.0f ? 1.0f / vmax : 0.0f;  // powers of two
-    if (__any(alpha != 1.0f) || vmax != ref) {
-      const float f = alpha * (ref * inv);
+    if (__any(alpha != 1.0f)) {
 #pragma unroll
-      for (int b = 0; b < VB; ++b) acc[b] *= f;
+      for (int b = 0; b < VB; ++b) acc[b] *= alpha;
       l *= alpha;
     }
     m = mx;
-    ref = vmax;
-    h8_t ph[2], pl[2];
+    // (scaled and shifted with one rounding, so the largest weights carry next
+    // to none: it makes up for the output's twelve a tile)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float p = __builtin_amdgcn_exp2f(s[i] - base + 14.0f);
-      l += p;
-      const float w = p * (vsc[i >> 2] * inv);
-      const _Float16 h = (_Float16)w;
-      ph[i >> 3][i & 7] = h;
-      pl[i >> 3][i & 7] = (_Float16)(w - (float)h);
+    for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sl2, -base));
+    l += (((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]))) +
+         (((s[8] + s[9]) + (s[10] + s[11])) + ((s[12] + s[13]) + (s[14] + s[15])));
+    b8_t p[3][2];  // 16 keys each
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      b2_t w[3];
+      split3(s[2 * j], s[2 * j + 1], w);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        p[i][j >> 2][2 * j & 7] = w[i].x;
+        p[i][j >> 2][(2 * j + 1) & 7] = w[i].y;
+      }
     }
+    // a tile's sum from zero, its small products first: one rounding a tile at
+    // the output's own size
 #pragma unroll
-    for (int b = 0; b < VB; ++b)
+    for (int b = 0; b < VB; ++b) {
+      f16v o = {};
+      b8_t vh[2];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const int at = v_unit(2 * u + half, 32 * b + col);
-        const h8_t vh = *(const h8_t*)&tl.v[0][32 * b + col][at];
-        const h8_t vl = *(const h8_t*)&tl.v[1][32 * b + col][at];
-        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph[u], acc[b], 0, 0, 0);
-        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[u], acc[b], 0, 0, 0);
-        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[u], acc[b], 0, 0, 0);
+        vh[u] = *(const b8_t*)&tl.v[0][32 * b + col][at];
+        const b8_t vm = *(const b8_t*)&tl.v[1][32 * b + col][at];
+        const b8_t vl = *(const b8_t*)&tl.v[2][32 * b + col][at];
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vl, p[0][u], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh[u], p[2][u], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vm, p[1][u], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vm, p[0][u], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh[u], p[1][u], o, 0, 0, 0);
       }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh[u], p[0][u], o, 0, 0, 0);
+      acc[b] += o;
+    }
+  }
+  const int met = __any(!(largest < 0x1p127f));
+  int* again = (int*)split_smem;
+  __syncthreads();  // every wave is done with the tile
+  if (lane == 0) again[wave] = met;
+  __syncthreads();
+  if ((again[0] | again[1] | again[2] | again[3]) != 0) {
+    constexpr int QT = 16 / GP;
+    __syncthreads();
+    for (int r = r0; r < min(r0 + kSplitRows / GP, a.rows); r += QT) {
+      prefill_tile<HD, GP, false>(a, r / QT, kvh, (float*)split_smem);
+      __syncthreads();  // (the next tile reuses the LDS)
+    }
+    return;
   }
   if (!live) return;
-  const float f = ref / xor32_sum(l);
+  const float f = xor32_sum(l);
   float* out = a.out + (size_t)qr * a.out_stride + (size_t)(kvh * G + qh) * HD;
 #pragma unroll
   for (int b = 0; b < VB; ++b)
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      *(f4_t*)(out + 32 * b + 8 * q + 4 * half) =
-          f4_t{acc[b][4 * q] * f, acc[b][4 * q + 1] * f, acc[b][4 * q + 2] * f, acc[b][4 * q + 3] * f};
+    for (int i = 0; i < 4; ++i)
+      *(f4_t*)(out + 32 * b + 8 * i + 4 * half) =
+          f4_t{acc[b][4 * i] / f, acc[b][4 * i + 1] / f, acc[b][4 * i + 2] / f, acc[b][4 * i + 3] / f};
 }
 
 // e^(s - m) for s <= m as 2^h (1 + f ln 2), h + f = (s - m) log2 e with h the
@@ -2180,15 +2245,17 @@ bool prefill_attention_supported(int hd, int group) {
 template <int HD, int GP>
 static hipError_t prefill_launch(const AttnArgs& a, hipStream_t stream) {
   if constexpr (HD <= 128) {
-    // 128-row workgroups once they cover 3/8 of the CUs (2 layers of hidden
-    // 3584, FFN 9472, 28 heads on 4: 400 tokens, 100 workgroups, 532 -> 521
-    // us; 600 670 -> 630; 1000 1152 -> 995; 256 tokens, 64 workgroups, 360 ->
-    // 365, so those keep the 16-row tiles)
-    const int groups = (a.rows * GP + kPairRows - 1) / kPairRows * a.n_kv;
-    if (8 * groups >= 3 * device_cus() &&
+    // 128-row workgroups once they cover 11/16 of the CUs (head_dim 64: 3/4).
+    // us, 16-row fp32 tiles -> this, groups of 1 to 16, after 0 to 6000
+    // positions: at head_dim 128 144 workgroups 1.2 times faster to 5 % slower,
+    // 160 1.3 times to 2 %, 192 1.12 to 1.45 times (28 heads on 4: 768 tokens
+    // 94 -> 79, 2000 444 -> 223); at 64 160 workgroups 1.15 times to 15 %
+    // slower, 192 1.3 times to 3 % (16 heads on 16: 1536 tokens 111 -> 96).
+    const int groups = (a.rows * GP + kSplitRows - 1) / kSplitRows * a.n_kv;
+    if (16 * groups >= (HD == 64 ? 12 : 11) * device_cus() &&
         (uint64_t)a.max_seq * a.n_kv * HD * 4 < (1ull << 31)) {  // 31-bit offsets
-      const auto kernel = attn_pair_kernel<HD, GP>;
-      const size_t lds = 2 * sizeof(PairTile<HD>);
+      const auto kernel = attn_split_kernel<HD, GP>;
+      const size_t lds = split_lds_bytes<HD>();
       const hipError_t e = allow_dynamic_lds((const void*)kernel, lds);
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL(kernel, dim3(groups), dim3(256), lds, stream, a);

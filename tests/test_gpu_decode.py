@@ -856,11 +856,11 @@ def test_prefill_qwen2_7b_layer_at_full_size(pkg, oracle, cuda, qtype):
     assert np.abs(got - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-6
 
 
-# Long prompts whose 128-row attention workgroups cover 3/8 of the CUs run on fp16 pairs; the same
-# prompt in shorter pieces keeps the fp32 MFMA tiles. Ragged lengths, a past that begins inside a tile
-# and whose values span twelve decades, groups padded from 1, 3, 7 and 12 heads.
+# The same prompt whole and in pieces short enough for the fp32 tiles: whole logits and caches, a past whose values
+# span twelve decades (row by row: the two tests below).
 @pytest.mark.parametrize("hd,n_heads,n_kv,n,start", [(128, 28, 4, 413, 70), (64, 8, 8, 1545, 0), (128, 24, 2, 801, 33),
-                                                     (64, 12, 4, 1001, 5), (128, 4, 4, 3100, 1)])
+                                                     (64, 12, 4, 1001, 5), (128, 4, 4, 3100, 1), (128, 28, 4, 701, 70),
+                                                     (64, 16, 16, 1545, 0), (128, 8, 8, 2801, 1)])
 def test_prefill_long_prompt_pair_attention(pkg, cuda, hd, n_heads, n_kv, n, start):
     import mini_llama_amd.decode as dec
     from synthetic import synth
@@ -882,8 +882,126 @@ def test_prefill_long_prompt_pair_attention(pkg, cuda, hd, n_heads, n_kv, n, sta
         return logits.clone(), dm.keys.clone(), dm.values.clone()
 
     whole, pieces = run(n), run(180)
-    for a, b in zip(whole, pieces):  # fp32 Linears both times: only sums in other orders
+    for a, b in zip(whole, pieces):  # fp32 Linears both times; scores and weighted sums to fp32, in other orders
         assert float((a - b).abs().max()) <= 3e-5 * float(b.abs().max())
+
+
+# Long prompts whose 128-row attention workgroups cover 11/16 of the CUs (head_dim 64: 3/4) run on bf16 triples, the
+# last two on the fp32 tiles. Ragged lengths, a past that begins inside a tile, groups padded from 1, 2, 3, 7 and 12
+# heads.
+LONG_PROMPTS = [(128, 28, 4, 701, 70), (64, 16, 16, 1545, 0), (128, 24, 2, 801, 33), (64, 12, 4, 1601, 5),
+                (128, 8, 8, 2801, 1), (128, 16, 8, 1350, 40), (128, 28, 4, 413, 70), (64, 12, 4, 1001, 5)]
+
+
+class AttentionRows:
+    """A two-layer model whose second layer's V rows are the first layer's attention outputs (of the first query head
+    of every kv head, normalised): wo copies them into columns of x that the embedding leaves at zero, the FFN adds
+    nothing, wv copies them out. wk is those heads' wq, so their rotated queries are the K rows of the cache. Token 1
+    has values of about 1e9, token 2 NaN everywhere."""
+    D = 256
+
+    def __init__(self, cuda, hd, n_heads, n_kv, n, start, same_heads=False):
+        """same_heads: every head of a group has the first one's queries (a NaN in another head's output would meet
+        wo's zeros)."""
+        import mini_llama_amd.decode as dec
+        import torch
+        kvd, dim = n_kv * hd, self.D + n_kv * hd
+        g = torch.Generator(device=cuda).manual_seed(n)
+        first = (torch.arange(n_kv) * (n_heads // n_kv))[:, None] * hd + torch.arange(hd)
+        first = first.reshape(-1).to(cuda)
+
+        def f32(t):
+            return {"type": "f32", "shape": tuple(t.shape), "data": t}
+
+        wq = torch.randn((n_heads * hd, dim), generator=g, device=cuda) * 0.5 / 16
+        wv = torch.randn((kvd, dim), generator=g, device=cuda) / 16
+        if same_heads:
+            wq = wq[first].view(n_kv, 1, hd, dim).expand(-1, n_heads // n_kv, -1, -1).reshape(-1, dim).contiguous()
+        wq[:, 0] = 0.0
+        wv[:, 0] *= 1e9  # column 0 is token 1's
+        out = torch.zeros((dim, n_heads * hd), device=cuda)
+        out[self.D + torch.arange(kvd, device=cuda), first] = 1.0
+        pick = torch.zeros((kvd, dim), device=cuda)
+        pick[torch.arange(kvd, device=cuda), self.D + torch.arange(kvd, device=cuda)] = 1.0
+        one = torch.ones(dim, device=cuda)
+        layers = [{"attention_norm": one, "ffn_norm": one, "wq": f32(wq), "wk": f32(wq[first].contiguous()),
+                   "wv": f32(v), "wo": f32(out), "w_gate": f32(torch.zeros((64, dim), device=cuda)),
+                   "w_up": f32(torch.zeros((64, dim), device=cuda)), "w_down": f32(torch.zeros((dim, 64), device=cuda))}
+                  for v in (wv, pick)]
+        emb = torch.randn((300, dim), generator=g, device=cuda)
+        emb[:, self.D:] = 0.0
+        emb[:, 0] = 0.0
+        emb[1, 0] = 1.0
+        emb[2] = math.nan
+        cfg = dict(vocab_size=300, dim=dim, hidden_dim=64, n_layers=2, n_heads=n_heads, n_kv_heads=n_kv, head_dim=hd,
+                   max_seq_len=3200, rope_type=1, rope_theta=1e4, rms_norm_eps=1e-5)
+        self.dm = dec.DecodeModel({"config": cfg, "token_embedding": emb, "final_norm": one,
+                                   "lm_head": f32(torch.zeros((300, dim), device=cuda)), "layers": layers}, device=cuda)
+        self.emb, self.n, self.start, self.hd = emb, n, start, hd
+        past = (start, n_kv, hd)
+        self.dm.keys[0, :start] = torch.randn(past, generator=g, device=cuda) * 0.5
+        self.dm.values[0, :start] = torch.randn(past, generator=g, device=cuda) * 10.0 ** torch.randint(
+            -9, 3, (start, n_kv, 1), generator=g, device=cuda)
+        self.tokens = np.random.default_rng(n).integers(3, 300, n)
+
+    def run(self):
+        """(the second layer's V rows, what they are in 64 bits, bound of the difference)"""
+        import torch
+        n, start, end = self.n, self.start, self.start + self.n
+        self.dm.prefill(self.tokens, start)
+        k, v = self.dm.keys[0, :end].double(), self.dm.values[0, :end].double()
+        hidden = torch.arange(end, device=k.device)[None, :] > start + torch.arange(n, device=k.device)[:, None]
+        outs, sizes = [], []
+        for h in range(k.shape[1]):
+            score = (k[start:, h] @ k[:, h].t().contiguous()) / self.hd ** 0.5
+            p = torch.softmax(score.masked_fill(hidden, -math.inf), dim=1)
+            vis = v[:, h].nan_to_num(0.0, 0.0, 0.0)  # non-finite values through the masked sum below
+            out = p.nan_to_num(0.0) @ vis
+            out[p.isnan().any(dim=1)] = math.nan
+            for at in (~v[:, h].isfinite()).any(dim=1).nonzero().flatten().tolist():
+                rows = ~hidden[:, at]
+                out[rows] += p[rows, at, None] * torch.where(v[at, h].isfinite(), 0.0, v[at, h])
+            outs.append(out)
+            sizes.append(p.nan_to_num(0.0) @ vis.abs())
+        attn, size = torch.cat(outs, dim=1), torch.cat(sizes, dim=1)
+        x = self.emb[torch.from_numpy(self.tokens).to(k.device)].double()[:, :self.D]
+        rms = ((x.square().sum(dim=1) + attn.square().sum(dim=1)) / (self.D + attn.shape[1]) + 1e-5).sqrt()[:, None]
+        # scores of up to ~5 to 2^-22 each way, weights and sums in fp32; the norm to 1e-6
+        return self.dm.values[1, start:end].reshape(n, -1).double(), attn / rms, (2e-5 * size + 2e-6 * attn.abs()) / rms
+
+
+@pytest.mark.parametrize("hd,n_heads,n_kv,n,start", LONG_PROMPTS)
+def test_prefill_long_prompt_split_attention(pkg, cuda, hd, n_heads, n_kv, n, start):
+    """Every row to fp32 accuracy of its own sum of |weight x value|, whatever the values of keys it does not see or
+    hardly weighs: tokens with values 1e9 times the others' among the prompt, a past over twelve decades."""
+    m = AttentionRows(cuda, hd, n_heads, n_kv, n, start)
+    m.tokens[[20, 21, 100, 250, n - 3]] = 1
+    got, want, bound = m.run()
+    assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() / bound).max())
+
+
+@pytest.mark.parametrize("hd,n_heads,n_kv,n,start", LONG_PROMPTS)
+def test_prefill_long_prompt_non_finite(pkg, cuda, hd, n_heads, n_kv, n, start):
+    """Keys of -inf weigh 0, +inf and NaN give NaN, to the rows that see them. A NaN token reaches, of the rows before
+    it, at most those of its 16-row tile of (query, head) pairs, as with short prompts."""
+    import torch
+    m = AttentionRows(cuda, hd, n_heads, n_kv, n, start, same_heads=True)
+    at, tile = n // 2 + 3, 16 // (1 << (n_heads // n_kv - 1).bit_length())
+    m.tokens[at] = 2
+    if start > 3:
+        m.dm.keys[0, 2, 0, 3] = -math.inf
+        m.dm.keys[0, 3, n_kv - 1, hd - 1] = math.inf
+    got, want, bound = m.run()
+    free = at // tile * tile
+    nan = want[:free].isnan()
+    assert torch.equal(got[:free].isnan(), nan)
+    assert bool(((got - want).abs() <= bound)[:free][~nan].all())
+    assert bool(got[at:].isnan().all())
+    if start > 3:  # some rows meet the infinite keys with either sign
+        assert bool(nan.any()) and not bool(nan.all())
+        m.dm.values[0, 2, 0, 5] = math.inf
+        got, want, bound = m.run()
+        assert torch.equal(got[:free].isnan(), want[:free].isnan())
 
 
 def test_prefill_tiny_model_greedy(pkg, oracle, cuda):
