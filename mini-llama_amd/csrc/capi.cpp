@@ -73,7 +73,7 @@ bool uses_gemv(const mlq_weight* w, int m) {
 bool uses_rows(const mlq_weight* w, int m) {
   if (m < 2 || m > 16 || (m <= kGemvMaxRows ? gemv_split_set() : skinny_plan_set())) return false;
   if (!rows_supported(w->type, m, w->n, w->k)) return false;
-  return rows_faster(m, w->n, w->k) || (m <= kGemvMaxRows && !uses_gemv(w, m));
+  return rows_faster(w->type, m, w->n, w->k) || (m <= kGemvMaxRows && !uses_gemv(w, m));
 }
 
 }  // namespace

@@ -149,7 +149,7 @@ hipError_t launch_split_reduce(const float* part, float* y, int m, int n, int sp
 // weight tiles; no workspace. rows_faster: the shapes it takes from the
 // decode GEMV and the skinny GEMM.
 bool rows_supported(int type, int m, int n, int k);
-bool rows_faster(int m, int n, int k);
+bool rows_faster(int type, int m, int n, int k);
 hipError_t launch_rows(const mlq_weight& w, const float* x, float* y, int m, hipStream_t stream,
                        const Epilogue& epi = Epilogue());
 

@@ -424,20 +424,32 @@ size_t lds_limit() {
 }
 }  // namespace
 
-// Where streaming past a resident x beats a workgroup per tile (4 layers of a
-// 7B model, us, workgroup per tile against this kernel for the shapes past
-// the line): it starts later (all of x is converted before the first unit),
-// so with few tiles the others win (288 and 224 tiles, 4 rows of q4_0: 206
-// with them left to the GEMV, 217 without).
-//  - 5..16 rows: more than 5/4 tiles per CU (8 rows of q4_0 578 -> 233, 16 rows
-//    of q8_0 501 -> 338; at hidden 2048, FFN 5632, 704 tiles, 115 -> 109 and
-//    191 -> 153).
-//  - 2..4 rows, whose x is small: 128 units per CU (4 rows of q4_0 307 -> 206;
-//    the 704-tile projections of hidden 2048 take 91.5 against 93.2).
-bool rows_faster(int m, int n, int k) {
+// Where streaming past a resident x beats a workgroup per tile. It starts later
+// (all of x is converted before the first unit), so a CU needs work enough to make
+// up for that. Both measured for 512..152064 weight rows and K 256..18944 (time
+// here over the workgroup per tile's, q8_0 / q4_0 / q4_1):
+//  - 2..4 rows, whose x is small: 128 units per CU (4 rows 0.7 to 1.0 there, of
+//    28672 x 4096 0.78 / 0.65 / 0.51). Not two rows of at most 8 groups (152064 x
+//    896 1.20 / 1.00 / 1.13), nor two or three of q8_0 where the GEMV's 16 waves
+//    share K evenly (two rows of 8192 x 8192 1.13, 65536 x 2048 1.22; 18944 x 3584
+//    0.94, 13824 x 5120 0.72).
+//  - 5..8 rows: more than 5/4 tiles per CU and 56 units per CU (6 rows 48, more
+//    40): 5 rows of 20480 x 1024, 40 units, 1.15 / 1.17 / 1.02, of 29000 x 896, 50,
+//    1.04 / 0.98 / 0.90; 8 rows of 8192 x 2048, 32, 1.07 / 1.00 / 0.89, of 14336 x
+//    1536, 42, 0.80 / 0.74 / 0.66, of 28672 x 4096 0.46 / 0.34 / 0.45.
+//  - 9..16 rows: more than 5/4 tiles per CU (16 of 5184 x 256 0.56 / 0.74 / 0.54, of
+//    18944 x 3584 0.50 / 0.59 / 0.49); in q4_0, whose skinny kernel runs two tiles per
+//    CU in one round, more than two of them past K 2048 (16 of 6144 x 4096 1.18, x
+//    2048 0.85, 11008 x 4096 0.74).
+bool rows_faster(int type, int m, int n, int k) {
   const Geometry geo = geometry(n, k);
-  if (m <= 4) return (int64_t)geo.nt * geo.g >= 128 * (int64_t)device_cus();
-  return 4 * (int64_t)geo.nt > 5 * (int64_t)device_cus();
+  const int64_t cus = device_cus(), units = (int64_t)geo.nt * geo.g;
+  if (m <= 4)
+    return units >= 128 * cus && !(m == 2 && geo.g <= 8) &&
+           !(m <= 3 && type == MLQ_Q8_0 && geo.g % 16 == 0);
+  if (4 * (int64_t)geo.nt <= 5 * cus) return false;
+  if (m <= 8) return units >= std::max(40, 8 * (12 - m)) * cus;
+  return type != MLQ_Q4_0 || geo.nt > 2 * cus || geo.g <= 16;
 }
 
 bool rows_supported(int type, int m, int n, int k) {

@@ -751,13 +751,14 @@ def test_cpp_interface_tests(pkg):
 
 
 # ---- 2..16 rows with x resident in LDS (rows.hip) ---------------------------------------------------
-# 5..16 rows from 321 weight tiles on, 2..4 rows from 32768 units on, and rows too long for the GEMV's
-# staging: runs of units shorter than a tile, whole tiles inside a run, uneven tile counts, the longest
+# 9..16 rows from 321 weight tiles on, 5..8 rows with 10240 to 14336 units, 2..4 rows from 32768 units on, and rows
+# too long for the GEMV's staging (the first shapes of 5 and 8 rows lie below those lines): runs of units shorter than a tile, whole tiles inside a run, uneven tile counts, the longest
 # K of each row count, ragged K and N, the padded row counts' edges.
 @pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("m,n,k", [(5, 5137, 100), (8, 5136, 132), (9, 5152, 36), (16, 5121, 4100), (12, 8208, 4864),
                                    (8, 9001, 4736), (16, 40000, 256), (2, 8209, 8196), (3, 16401, 4096),
                                    (4, 16400, 4228), (2, 3584, 17408), (3, 640, 9216), (6, 100, 4864),
+                                   (5, 16400, 2052), (6, 20481, 1292), (7, 8209, 2560), (8, 5136, 4100),
                                    # x in two, three and five pieces
                                    (4, 4096, 14336), (8, 100, 9860), (5, 4090, 18948), (2, 48, 40004)])
 def test_resident_rows(pkg, cuda, qtype, m, n, k):
@@ -773,8 +774,9 @@ def test_resident_rows(pkg, cuda, qtype, m, n, k):
     w64, x64 = pkg.dequantize(tw).double(), x.double()
     ref = x64 @ w64.t().contiguous() + bias.double()
     size = x64.abs() @ w64.abs().t().contiguous() + bias.abs().double()
-    # up to 8 rows (where the longest x fits): x to 2^-22, fp32 sums; more: x and W rounded to fp16 once
-    grow = 2.0 ** -20 if m <= 8 and pkg.workspace_bytes(tw, m) == 0 else 2.0 ** -10
+    # up to 8 rows: x to 2^-22, fp32 sums, no workspace; more: x and W rounded to fp16 once
+    grow = 2.0 ** -20 if m <= 8 else 2.0 ** -10
+    assert m > 8 or pkg.workspace_bytes(tw, m) == 0
     y = pkg.linear(tw, x, bias=bias).double()
     assert bool(((y - ref).abs() <= grow * size).all())
     if n % 16 == 0:
