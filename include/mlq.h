@@ -138,10 +138,12 @@ int mlq_quantize_act_q8_0(const float* x, int rows, int row_size, void* out,
 /* ---------------------------------------------------------------------- */
 
 /* Tiled weight (from the upload path). Picks the kernel family by m:
- *  m = 1..8 (decode): HBM-streaming GEMV, fp32-class accuracy; with many
- *    weight tiles, or an x too long for its staging, 2..8 (and with many
- *    tiles 9..16) rows stream past an x kept in LDS, same accuracy for their
- *    row count. One row:
+ *  m = 1..8 (decode): HBM-streaming GEMV, fp32-class accuracy. With many
+ *    weight tiles, or an x too long for its staging, 2..8 rows stream past an
+ *    x kept in LDS, same accuracy (k % 4 == 0; on up to one 16-row tile per
+ *    CU any k, on more up to k = 20224 / 10112 / 4992 for 2 / 4 / 8 rows,
+ *    q4_1 19584 / 9728 / 4864); past both they run as 9..64 rows do, in fp16.
+ *    One row:
  *    activations as integers (22 bits below the largest |x| of each K
  *    slice, three fp16 digits), codes fed with their fp16 bias and the
  *    bias removed on the matrix core, every block sum exact; several rows
@@ -158,9 +160,10 @@ int mlq_linear(const mlq_weight* w, const float* x, float* y, int m,
 /* Device workspace bytes mlq_linear_ws needs for m activation rows with
  * weight w (*bytes = 0 when the kernels for that shape need none: the decode
  * GEMV and the resident-x kernel (most calls of 2..8 rows), and 9..16 rows
- * with k <= 6144, k % 4 == 0, whose skinny kernel reads fp32 x itself). The skinny (17..64 rows, or longer rows) and prefill
- * GEMMs use it for a one-pass fp16 copy of x, which halves the activation
- * bytes their stages move; both also for fp32 partial outputs when they
+ * with k <= 6144, k % 4 == 0, whose skinny kernel reads fp32 x itself). The
+ * skinny (17..64 rows, or longer rows) and prefill GEMMs use it for a
+ * one-pass fp16 copy of x, which halves the activation bytes their stages
+ * move; both also for fp32 partial outputs when they
  * split K across workgroups (shapes with few output tiles). The size
  * depends on the shape, the split-K overrides and the device's
  * compute-unit count. */

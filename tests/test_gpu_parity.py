@@ -788,6 +788,59 @@ def test_resident_rows(pkg, cuda, qtype, m, n, k):
         assert bool(((y - torch.nn.functional.silu(gate) * up).abs() <= slack).all())
 
 
+# An infinite or NaN activation makes its own row's outputs non-finite (F32: what the fp32 products give) and leaves
+# every other row's bits alone: resident-x rows (fp32-class, in pieces, fp16), 17..64 rows past LDS, F32 tiles and rows.
+@pytest.mark.parametrize("qtype,m,n,k", [
+    ("q8_0", 8, 9001, 2436), ("q4_1", 4, 16400, 4228), ("q4_1", 6, 96, 9860), ("q4_0", 16, 16400, 260),
+    ("q4_1", 11, 5136, 132), ("q8_0", 40, 20480, 260), ("q4_0", 64, 20501, 132), ("q4_1", 17, 20480, 516),
+    ("f32", 769, 1040, 288), ("f32", 769, 1040, 3076), ("f32", 33, 64, 288), ("f32", 12, 100, 1001)])
+def test_non_finite_rows(pkg, cuda, qtype, m, n, k):
+    import torch
+    from synthetic import synth
+    _print_case(test="non_finite_rows", qtype=qtype, m=m, n=n, k=k)
+    g = torch.Generator(device=cuda).manual_seed(m + n + k)
+    if qtype == "f32":
+        w = torch.randn((n, k), generator=g, device=cuda)
+        tw = pkg.TiledWeight("f32", n, k, w.view(-1).view(torch.uint8), pkg.weight_layout("f32", n, k))
+    else:
+        tw = pkg.repack_device(qtype, synth.device_blocks(torch, g, qtype, n, k, 0.02, cuda).view(-1).view(torch.uint8), n, k)
+        w = pkg.dequantize(tw)
+    x = torch.randn((m, k), generator=g, device=cuda)
+    clean = pkg.linear(tw, x)
+    assert bool(clean.isfinite().all())
+    rows = torch.arange(m, device=cuda)
+    for row, col, value in ((0, 0, math.inf), (m - 1, k - 1, -math.inf), (m // 2, k // 2, math.nan)):
+        bad = x.clone()
+        bad[row, col] = value
+        y = pkg.linear(tw, bad)
+        assert torch.equal(y[rows != row], clean[rows != row]), (row, col, value)
+        if qtype != "f32":
+            assert not bool(y[row].isfinite().any()), (row, col, value)
+        elif math.isnan(value):
+            assert bool(y[row].isnan().all())
+        else:
+            assert torch.equal(y[row], value * w[:, col])
+
+
+# Up to 8 rows whose x is too long for the LDS: in pieces on at most a 16-row tile per CU, at fp32-class accuracy; on
+# more tiles, and with k % 4 != 0, as 9..64 rows run (x and W rounded to fp16 once).
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("m,n,k,exact", [(8, 4096, 9860, True), (8, 4112, 9860, False), (2, 4096, 24580, True),
+                                         (2, 4112, 24580, False), (8, 96, 9861, False)])
+def test_long_rows_accuracy(pkg, cuda, qtype, m, n, k, exact):
+    import torch
+    from synthetic import synth
+    _print_case(test="long_rows", qtype=qtype, m=m, n=n, k=k)
+    g = torch.Generator(device=cuda).manual_seed(m + n + k)
+    tw = pkg.repack_device(qtype, synth.device_blocks(torch, g, qtype, n, k, 0.02, cuda).view(-1).view(torch.uint8), n, k)
+    x = torch.randn((m, k), generator=g, device=cuda)
+    w64, x64 = pkg.dequantize(tw).double(), x.double()
+    ref, size = x64 @ w64.t().contiguous(), x64.abs() @ w64.abs().t().contiguous()
+    assert (pkg.workspace_bytes(tw, m) == 0) == exact
+    err = (pkg.linear(tw, x).double() - ref).abs()
+    assert bool((err <= (2.0 ** -20 if exact else 2.0 ** -10) * size).all())
+
+
 # Raw GGUF blocks on both sides of the lines between their two kernels, several tiles per workgroup (whole and shared), odd block counts (rows off
 # 4-byte boundaries), k % 4 != 0, a base off a 4-byte boundary, blocks of the last group past the row.
 @pytest.mark.parametrize("qtype", TYPES)
