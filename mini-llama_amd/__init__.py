@@ -234,8 +234,12 @@ def _stream(stream=None) -> int:
     if stream is not None:
         return stream.cuda_stream
     import torch
-    # the handle alone: building a Stream object takes 3 us, as long as a launch
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    # the handle alone where torch gives it: building a Stream object takes 3 us,
+    # as long as a launch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch.cuda.current_device())
 
 
 class TiledWeight:

@@ -240,3 +240,17 @@ def test_fixture_file_is_regenerable():
     assert committed["fp16_rounding"] == make_fixtures.tie_vectors()
     assert committed["reference_tests"] == json.loads(
         json.dumps(make_fixtures.reference_test_vectors()))
+
+
+def test_current_stream_handle(pkg, monkeypatch):
+    """torch's private raw handle is used where it exists, the public Stream object where it does not."""
+    import types
+
+    import torch
+    assert pkg._stream(types.SimpleNamespace(cuda_stream=11)) == 11
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=7))
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 100 + device, raising=False)
+    assert pkg._stream() == 103
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert pkg._stream() == 7
