@@ -29,10 +29,11 @@
 // K = 256; in the tiled kernel of 16 k from K = 1536 and of 32 k from K = 3072,
 // where the GEMV's own chains have grown past them (every chain that is cut
 // costs 16 additions per lane: 200 x 4096 x 4096 takes 91 us in chains of 8).
-// Modelled error, GEMV against tiled and skinny: K = 256 7.7e-8, 7.9e-8,
-// 7.9e-8; 512 8.8e-8, 8.4e-8, 8.4e-8; 1536 1.11e-7, 1.07e-7, 9.7e-8; 3072
-// 1.42e-7, 1.24e-7, 1.03e-7; 4096 1.55e-7, 1.25e-7, 1.07e-7
-// (chains of 32 k: 1.2e-7 at 256 and 512).
+// Measured error against 64 bits (normal inputs, 4096 W rows), GEMV against tiled
+// and skinny: K = 64 6.77e-8, 6.76e-8, 6.77e-8; 256 7.79e-8, 7.79e-8, 7.80e-8; 512
+// 8.57e-8, 8.36e-8, 8.24e-8; 1536 1.12e-7, 1.03e-7, 9.2e-8; 3072 1.42e-7, 1.27e-7,
+// 1.03e-7; 4096 1.59e-7, 1.30e-7, 1.10e-7; 15000 2.83e-7, 1.57e-7, 1.62e-7 (chains of
+// 32 k modelled 1.2e-7 at 256 and 512).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
