@@ -1020,8 +1020,10 @@ __device__ __forceinline__ void prefill_tile(const AttnArgs& a, int tile, int kv
   }
 }
 
+// (head_dim 128: at more than 256 registers one wave per SIMD instead of two takes
+// 62.6 us for 512 rows, 28 heads on 4, instead of 48)
 template <int HD, int GP>
-__global__ __launch_bounds__(prefill_waves(HD) * 64) void attn_prefill_kernel(AttnArgs a) {
+__global__ __launch_bounds__(prefill_waves(HD) * 64, HD <= 128 ? 2 : 1) void attn_prefill_kernel(AttnArgs a) {
   __shared__ __align__(16) float lds[prefill_lds_floats<HD>()];
   prefill_tile<HD, GP, true>(a, blockIdx.x, blockIdx.y, lds);
 }
@@ -2245,14 +2247,15 @@ bool prefill_attention_supported(int hd, int group) {
 template <int HD, int GP>
 static hipError_t prefill_launch(const AttnArgs& a, hipStream_t stream) {
   if constexpr (HD <= 128) {
-    // 128-row workgroups once they cover 11/16 of the CUs (head_dim 64: 3/4).
+    // 128-row workgroups once they cover 11/16 of the CUs (head_dim 64: 7/8).
     // us, 16-row fp32 tiles -> this, groups of 1 to 16, after 0 to 6000
-    // positions: at head_dim 128 144 workgroups 1.2 times faster to 5 % slower,
-    // 160 1.3 times to 2 %, 192 1.12 to 1.45 times (28 heads on 4: 768 tokens
-    // 94 -> 79, 2000 444 -> 223); at 64 160 workgroups 1.15 times to 15 %
-    // slower, 192 1.3 times to 3 % (16 heads on 16: 1536 tokens 111 -> 96).
+    // positions: at head_dim 128 176 workgroups 1.33 times faster to 2 %
+    // slower, 192 1.05 to 1.56 times (28 heads on 4: 768 tokens 93 -> 83, 2000
+    // 409 -> 217); at 64 192 workgroups 1.22 times to 11 % slower, 208 1.39
+    // times to 7 %, 224 1.0 to 1.41 times (16 heads on 16: 1792 tokens
+    // 122 -> 111).
     const int groups = (a.rows * GP + kSplitRows - 1) / kSplitRows * a.n_kv;
-    if (16 * groups >= (HD == 64 ? 12 : 11) * device_cus() &&
+    if (16 * groups >= (HD == 64 ? 14 : 11) * device_cus() &&
         (uint64_t)a.max_seq * a.n_kv * HD * 4 < (1ull << 31)) {  // 31-bit offsets
       const auto kernel = attn_split_kernel<HD, GP>;
       const size_t lds = split_lds_bytes<HD>();

@@ -860,7 +860,8 @@ def test_prefill_qwen2_7b_layer_at_full_size(pkg, oracle, cuda, qtype):
 # span twelve decades (row by row: the two tests below).
 @pytest.mark.parametrize("hd,n_heads,n_kv,n,start", [(128, 28, 4, 413, 70), (64, 8, 8, 1545, 0), (128, 24, 2, 801, 33),
                                                      (64, 12, 4, 1001, 5), (128, 4, 4, 3100, 1), (128, 28, 4, 701, 70),
-                                                     (64, 16, 16, 1545, 0), (128, 8, 8, 2801, 1)])
+                                                     (64, 16, 16, 1545, 0), (128, 8, 8, 2801, 1),
+                                                     (64, 16, 16, 1801, 0)])
 def test_prefill_long_prompt_pair_attention(pkg, cuda, hd, n_heads, n_kv, n, start):
     import mini_llama_amd.decode as dec
     from synthetic import synth
@@ -886,10 +887,10 @@ def test_prefill_long_prompt_pair_attention(pkg, cuda, hd, n_heads, n_kv, n, sta
         assert float((a - b).abs().max()) <= 3e-5 * float(b.abs().max())
 
 
-# Long prompts whose 128-row attention workgroups cover 11/16 of the CUs (head_dim 64: 3/4) run on bf16 triples, the
+# Long prompts whose 128-row attention workgroups cover 11/16 of the CUs (head_dim 64: 7/8) run on bf16 triples, the
 # last two on the fp32 tiles. Ragged lengths, a past that begins inside a tile, groups padded from 1, 2, 3, 7 and 12
 # heads.
-LONG_PROMPTS = [(128, 28, 4, 701, 70), (64, 16, 16, 1545, 0), (128, 24, 2, 801, 33), (64, 12, 4, 1601, 5),
+LONG_PROMPTS = [(128, 28, 4, 701, 70), (64, 16, 16, 1801, 0), (128, 24, 2, 801, 33), (64, 12, 4, 1801, 5),
                 (128, 8, 8, 2801, 1), (128, 16, 8, 1350, 40), (128, 28, 4, 413, 70), (64, 12, 4, 1001, 5)]
 
 
